@@ -1,0 +1,330 @@
+// The cell-per-wave Rodas3 attempt on cell programs (mechgen/cell_sched.py):
+// one wavefront integrates one cell whose LU and solve vector live in LDS
+// (fullchem: 53 KB, three cells per CU) and whose state, rate constants,
+// stage vectors and the LU's tail block live in the lanes' registers.
+//
+// What bounds it: the LDS round trips of the levels in front of the tail block
+// and the operand reads, two per FMA (about 2,600 LDS reads an attempt), with
+// one wave per SIMD to hide them.  Hence straight-line programs (no flags, no
+// loop control: 14.7k instructions, the operands of six steps in flight), sums
+// cut into 32-term chunks so that a 384-term row is not one lane's serial
+// chain, the last 34 rows -- a chain of pivots -- in registers, and the
+// reaction products in LDS over the tail block's slots (gathered from L2 they
+// cost 64 cache lines a step).  Measured on the 24x23x72 grid, cold step of
+// 39,744 cells: 537 ms with the block programs of wave_sched.py, 118 ms here;
+// 63 us an attempt and wave where it was 280 us; one cell's Integrate 9.2 ms
+// and 2.8 ms.
+//
+// Included by wave_solver.hip inside namespace gckpp.
+#pragma once
+
+typedef __attribute__((address_space(3))) double lds_double;
+
+// One wave's LDS block by byte offset; own: the block plus the lane's double.
+struct CellLds {
+  unsigned base, own, coef;
+  int lane;
+};
+__device__ __forceinline__ double cell_ld(unsigned off) { return *(const lds_double *)off; }
+__device__ __forceinline__ void cell_st(unsigned off, double v) { *(lds_double *)off = v; }
+
+// Block k of a program's words (four words a lane, 1 KB a block).
+__device__ __forceinline__ uint4 cell_word(const unsigned *w, int lane, int k) {
+  return *(const uint4 *)(w + (k * 64 + lane) * 4);
+}
+// True on the lanes of a constant mask (the mask goes straight into exec).
+__device__ __forceinline__ bool lanes_of(unsigned long long m) {
+  return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+// Lane l's value on every lane.
+__device__ __forceinline__ double bcast(double v, int l) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+  const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+  return __builtin_bit_cast(double, hi << 32 | lo);
+}
+// x / d from y = 1 / d (correctly rounded): Markstein's two-step quotient
+// (IBM J. Res. Dev. 34(1), 1990), the same double as x / d for finite
+// operands away from underflow, in three dependent FMAs where the division
+// sequence takes eleven instructions.  exact: the division itself.
+__device__ __forceinline__ double cell_div(double x, double d, double y, int exact) {
+  if (exact) return x / d;
+  const double q = x * y;
+  return fma(fma(-d, q, x), y, q);
+}
+
+#define LD(off) cell_ld(c.base + (off))
+#define ST(off, v) cell_st(c.base + (off), v)
+#define CF(off) cell_ld(c.coef + (off))
+#define LDL(off) cell_ld(c.own + (off))
+#define STL(off, v) cell_st(c.own + (off), v)
+#include "gen/cell_fullchem.h"
+
+// The cell programs of a mechanism that has them (Traits::TAIL > 0).
+template <class M> struct CellProg;
+template <> struct CellProg<Traits_fullchem> {
+  static constexpr int TAIL = cell_fullchem::TAIL, ROWS = cell_fullchem::ROWS;
+  static constexpr int NCOEF = cell_fullchem::NCOEF, SIZE = cell_fullchem::SIZE;
+  static constexpr int X0 = cell_fullchem::X0, CELLS = cell_fullchem::CELLS;
+  static __device__ __forceinline__ void fun(const CellLds &c, const double (&R)[ROWS]) {
+    cell_fullchem::cell_fun(c, R);
+  }
+  static __device__ __forceinline__ void jac(const CellLds &c, const double (&R)[ROWS], double diag,
+                                             bool &bad) {
+    cell_fullchem::cell_jac(c, R, diag, bad);
+  }
+  static __device__ __forceinline__ void lu(const CellLds &c, double (&T)[TAIL], double &ud,
+                                            double &yd) {
+    cell_fullchem::cell_lu(c, T, ud, yd);
+  }
+  static __device__ __forceinline__ void solve(const CellLds &c, const double (&T)[TAIL], double ud,
+                                               double yd) {
+    cell_fullchem::cell_solve(c, T, ud, yd);
+  }
+  static __device__ int rx(int i) { return cell_fullchem::rx[i]; }
+  static __device__ double coef(int i) { return cell_fullchem::coef[i]; }
+  static __device__ __forceinline__ void constants(const CellLds &c) {
+    if (c.lane == 0) {
+      ST(8 * cell_fullchem::ZERO, 0.0);
+      ST(8 * cell_fullchem::ONE, 1.0);
+      ST(8 * cell_fullchem::NEG, -1.0);
+    }
+  }
+};
+
+// What a lane keeps of its wave's cell between attempts: the rate constants
+// of its reactions, and of species lane + 64 k the concentration, Fcn0 and
+// the tolerances.
+template <class M>
+struct CellState {
+  static constexpr int KS = (M::NVAR + 63) / 64;
+  double R[CellProg<M>::ROWS], Y[KS], F0[KS], at[KS], rt[KS];
+};
+
+// Fixed species, rate constants and tolerances of the cell; Y is the
+// caller's.
+template <class M>
+__device__ __forceinline__ void cell_load(const IntegrateArgs &a, const CellLds &c, int64_t cell,
+                                          CellState<M> &s) {
+  using P = CellProg<M>;
+  wave_sync();
+  P::constants(c);
+  if (c.lane < M::NFIX)
+    STL(8 * (P::X0 + M::NVAR), a.conc[(int64_t)(M::NVAR + c.lane) * a.cstride + cell]);
+#pragma unroll
+  for (int u = 0; u < P::ROWS; ++u)
+    s.R[u] = a.rconst[(int64_t)P::rx(u * 64 + c.lane) * a.rstride + cell];
+#pragma unroll
+  for (int k = 0; k < CellState<M>::KS; ++k) {
+    const int i = c.lane + 64 * k < M::NVAR ? c.lane + 64 * k : M::NVAR - 1;
+    s.at[k] = a.atol[a.prm.vectol ? i : 0];
+    s.rt[k] = a.rtol[a.prm.vectol ? i : 0];
+  }
+  wave_sync();
+}
+
+template <class M>
+__device__ __forceinline__ void cell_begin(const IntegrateArgs &a, const CellLds &c, int64_t cell,
+                                           CellState<M> &s) {
+  cell_load<M>(a, c, cell, s);
+#pragma unroll
+  for (int k = 0; k < CellState<M>::KS; ++k) {
+    const int i = c.lane + 64 * k < M::NVAR ? c.lane + 64 * k : M::NVAR - 1;
+    s.Y[k] = a.conc[(int64_t)i * a.cstride + cell];
+  }
+}
+
+// Continues a handed-off cell (see state_resume).
+template <class M>
+__device__ __forceinline__ void cell_resume(const IntegrateArgs &a, const Handoff &ho,
+                                            const CellLds &c, int64_t cell, int64_t idx,
+                                            CellState<M> &s) {
+  cell_load<M>(a, c, cell, s);
+#pragma unroll
+  for (int k = 0; k < CellState<M>::KS; ++k) {
+    const int i = c.lane + 64 * k < M::NVAR ? c.lane + 64 * k : M::NVAR - 1;
+    s.Y[k] = ho.rec[(HO_FIELDS + i) * ho.cap + idx];
+  }
+}
+
+template <class M>
+__device__ __forceinline__ void cell_finish(const IntegrateArgs &a, const CellLds &c, int64_t cell,
+                                            const CellState<M> &s) {
+#pragma unroll
+  for (int k = 0; k < CellState<M>::KS; ++k) {
+    const int i = c.lane + 64 * k;
+    const double v = a.clip_out ? (s.Y[k] > 0.0 ? s.Y[k] : 0.0) : s.Y[k];
+    if (i < M::NVAR) a.conc[(int64_t)i * a.cstride + cell] = v;
+  }
+  if (a.clip_out && c.lane < M::NFIX) {
+    const double v = LDL(8 * (CellProg<M>::X0 + M::NVAR));
+    a.conc[(int64_t)(M::NVAR + c.lane) * a.cstride + cell] = v > 0.0 ? v : 0.0;
+  }
+}
+
+// One Rodas3 attempt of the wave's cell (lane_attempt's algorithm and order
+// of operations); true when the cell is done (S.ierr then holds IERR).
+template <class M>
+__device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellLds &c, int64_t cell,
+                                             WaveState &S, CellState<M> &cs) {
+  using P = CellProg<M>;
+  constexpr int N = M::NVAR, KS = CellState<M>::KS;
+  const RosParams &prm = a.prm;
+  const double Tend = prm.Tend, dir = prm.direction;
+  // the lane's species of a vector to X and back
+  auto put = [&](const double (&v)[KS]) {
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      if (64 * (k + 1) <= N || c.lane + 64 * k < N) STL(8 * (P::X0 + 64 * k), v[k]);
+    wave_sync();
+  };
+  auto get = [&](double (&v)[KS]) {
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      v[k] = 64 * (k + 1) <= N || c.lane + 64 * k < N ? LDL(8 * (P::X0 + 64 * k)) : 0.0;
+    wave_sync();
+  };
+  if (S.newStep) {
+    const bool more = (dir > 0) ? ((S.T - Tend) + prm.roundoff <= 0.0) : ((Tend - S.T) + prm.roundoff <= 0.0);
+    if (!more) return true;
+    if (S.st[2] > prm.max_steps) { S.ierr = -6; return true; }
+    if ((S.T + 0.1 * S.H) == S.T || S.H <= prm.roundoff) { S.ierr = -7; return true; }
+    S.H = min_f(S.H, fabs(Tend - S.T));
+  }
+  double K0[KS], K1[KS], K2[KS], K3[KS], T[P::TAIL], ud = 1.0, yd = 1.0, dH = 0.0;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) K0[k] = K1[k] = K2[k] = K3[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < P::TAIL; ++k) T[k] = 0.0;
+  // s = -1: Fcn0 of a new step; s = 0: the matrix and its LU; s = 0..3: the
+  // stages.  A loop, so that the programs are inlined once.
+#pragma unroll 1
+  for (int s = S.newStep ? -1 : 0; s < 4; ++s) {
+    double v[KS];
+    if (s < 0 || s >= 2) {
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        v[k] = cs.Y[k];
+        if (s >= 2) v[k] = fma(2.0, K0[k], v[k]);
+        if (s == 3) v[k] = fma(1.0, K2[k], v[k]);
+      }
+      put(v);
+      P::fun(c, cs.R);
+      get(v);
+      S.st[0] += s >= 0 || prm.autonomous ? 1 : 2;
+      if (s < 0) {
+        S.st[1] += 1;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) cs.F0[k] = v[k];
+        continue;
+      }
+    } else {
+      if (s == 0) {
+        int nconsec = 0;
+        bool singular = true;
+        while (singular) {
+          put(cs.Y);
+          bool bad = false;
+          P::jac(c, cs.R, 1.0 / (dir * S.H * kRosGamma1), bad);
+          const bool ising = __ballot(bad) != 0;
+          if (!ising) P::lu(c, T, ud, yd);
+          S.st[5] += 1;
+          if (!ising) {
+            singular = false;
+          } else {
+            S.st[7] += 1;
+            ++nconsec;
+            if (nconsec <= 5) S.H *= 0.5;
+            else break;
+          }
+        }
+        if (singular) { S.ierr = -8; return true; }
+        dH = dir * S.H;
+      }
+#pragma unroll
+      for (int k = 0; k < KS; ++k) v[k] = cs.F0[k];
+    }
+    if (s > 0) {
+      const double c0 = (s == 1 ? 4.0 : 1.0) / dH, c1 = -1.0 / dH, c2 = -(8.0 / 3.0) / dH;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        v[k] = fma(c0, K0[k], v[k]);
+        if (s >= 2) v[k] = fma(c1, K1[k], v[k]);
+        if (s == 3) v[k] = fma(c2, K2[k], v[k]);
+      }
+    }
+    put(v);
+    P::solve(c, T, ud, yd);
+    get(v);
+    S.st[6] += 1;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      if (s == 0) K0[k] = v[k];
+      else if (s == 1) K1[k] = v[k];
+      else if (s == 2) K2[k] = v[k];
+      else K3[k] = v[k];
+    }
+  }
+  const double H = S.H;
+  // Ynew and the error norm: a lane's terms in species order, then the 64
+  // lanes' sums in lane order
+  double yn[KS], part = 0.0;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    yn[k] = fma(1.0, K3[k], fma(1.0, K2[k], fma(2.0, K0[k], cs.Y[k])));
+    const double ye = fma(1.0, K3[k], 0.0);
+    const double ymax = max_f(fabs(cs.Y[k]), fabs(yn[k]));
+    const double q = ye / (cs.at[k] + cs.rt[k] * ymax);
+    if (64 * (k + 1) <= N || c.lane + 64 * k < N) part = fma(q, q, part);
+  }
+  wave_sync();
+  STL(8 * P::X0, part);
+  wave_sync();
+  double err = 0.0;
+#pragma unroll 1
+  for (int l = 0; l < 64; l += 16) {
+    double q[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) q[u] = LD(8 * (P::X0 + l + u));
+#pragma unroll
+    for (int u = 0; u < 16; ++u) err += q[u];
+  }
+  err = max_f(sqrt(err / N), 1.0e-10);
+  const double fac = min_f(prm.FacMax, max_f(prm.FacMin, prm.FacSafe / pow(err, 1.0 / kRosELO)));
+  S.Hnew = H * fac;
+  if (a.hlog && S.st[2] < a.hlog_n && c.lane == 0) {
+    a.hlog[(int64_t)(2 * S.st[2]) * a.ncell + cell] = (float)H;
+    a.hlog[(int64_t)(2 * S.st[2] + 1) * a.ncell + cell] = (float)err;
+  }
+  S.st[2] += 1;
+  if (err <= 1.0 || H <= prm.Hmin) {
+    S.st[3] += 1;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) cs.Y[k] = prm.clip_negative ? max_f(yn[k], 0.0) : yn[k];
+    S.T = S.T + dir * H;
+    S.Hnew = max_f(prm.Hmin, min_f(S.Hnew, prm.Hmax));
+    if (S.rejLast) S.Hnew = min_f(S.Hnew, H);
+    S.Hexit = H;
+    S.Texit = S.T;
+    S.HnewAcc = S.Hnew;
+    S.rejLast = S.rejMore = false;
+    S.H = S.Hnew;
+    S.newStep = true;
+  } else {
+    if (S.rejMore) S.Hnew = H * prm.FacRej;
+    S.rejMore = S.rejLast;
+    S.rejLast = true;
+    S.H = S.Hnew;
+    if (S.st[3] >= 1) S.st[4] += 1;
+    S.newStep = false;
+  }
+  return false;
+}
+
+#undef LD
+#undef ST
+#undef CF
+#undef LDL
+#undef STL

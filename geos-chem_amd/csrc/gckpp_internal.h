@@ -81,6 +81,7 @@ struct PersistArgs {
   double *work;          // [nblocks][slot_fields][64]
   int64_t slot_fields;
   unsigned int *counter; // work-stealing counter, or null (one cell per lane)
+  int64_t nwaves;        // waves of the launch (set by launch_persist)
   Handoff ho;
 };
 
@@ -139,7 +140,14 @@ constexpr int PERSIST_WAVE_VARIANT = 7;  // one wave per cell (wave_solver.hip)
 int persist_variant_info(int variant, int *U, int *W);
 int persist_variant_cache(int variant);  // operand-cache slots per lane (0: none)
 int persist_variant_seg(int variant);  // 0 lane per cell, 1 with flat segments, 2 wave per cell
-const void *wave_kernel(int qset);     // the cell-per-wave kernel (64 threads per workgroup)
+// The cell-per-wave kernel: the most waves a workgroup may have, and the
+// doubles of LDS a workgroup and each of its waves need.
+struct WaveKernel {
+  const void *fn;
+  int max_wpb, lds_group, lds_wave;
+  size_t lds(int wpb) const { return sizeof(double) * (size_t)(lds_group + wpb * lds_wave); }
+};
+WaveKernel wave_kernel(int qset);
 int64_t wave_scratch_fields(int qset);  // its global scratch per wave, fields of 64 doubles
 int64_t persist_slot_fields(int qset);                   // doubles per lane slot
 int64_t persist_resident_waves(int qset, int variant, int wpb);  // 0 on error

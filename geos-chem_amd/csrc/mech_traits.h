@@ -28,6 +28,9 @@ enum { WP_FV = 0, WP_JV = 1, WP_LU = 2, WP_SF = 3, WP_SB = 4 };
     static constexpr int NSPEC = mech_##NS::NSPEC, NREACT = mech_##NS::NREACT; \
     static constexpr int LU_NZ = mech_##NS::LU_NZ, NPART = mech_##NS::NPART;   \
     static constexpr int RX_MAX = mech_##NS::RX_MAX;                           \
+    static constexpr int TAIL = mech_##NS::TAIL;                               \
+    static __device__ int cr_hd(int i) { return mech_##NS::cr_hd[i]; }         \
+    static __device__ int fw_hd(int i) { return mech_##NS::fw_hd[i]; }         \
     /* entries of the Jacobian-term and Crout-term tables */                   \
     static constexpr int NJV_TAB = sizeof(mech_##NS::jv_b) / sizeof(int);      \
     static constexpr int NCR_TAB = sizeof(mech_##NS::cr_l) / sizeof(int);      \

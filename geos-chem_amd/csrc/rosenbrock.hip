@@ -103,6 +103,25 @@ __device__ __forceinline__ double gather_fma(int t0, int t1, double acc, W w, V 
   return acc;
 }
 
+// The same sum in the order of the cell programs (mechgen/cell_sched.py) for
+// a mechanism that has them: chunks of 32 terms, the first from init and the
+// others from +0.0, added in order; the terms from th on, which belong to the
+// tail block, follow one by one.  The cell-per-wave solver computes a sum's
+// chunks on different lanes, and every solver rounds alike.
+constexpr int kChunk = 32;
+template <class M, int U, class W, class V>
+__device__ __forceinline__ double gather_sum(int t0, int th, int t1, double init, W w, V v) {
+  if constexpr (M::TAIL == 0) {
+    return gather_fma<U>(t0, t1, init, w, v);
+  } else {
+    double acc = gather_fma<U>(t0, min(t0 + kChunk, th), init, w, v);
+#pragma unroll 1
+    for (int t = t0 + kChunk; t < th; t += kChunk)
+      acc = acc + gather_fma<U>(t, min(t + kChunk, th), 0.0, w, v);
+    return gather_fma<U>(th, t1, acc, w, v);
+  }
+}
+
 // Segment sums over a flat term list: segment s (s0 <= s < s1) covers terms
 // [sp(s), sp(s+1)); its value, sum_t w(t)*v(t) accumulated in term order from
 // 0, goes to fin(s, value) when the segment ends (empty segments give 0).
@@ -206,7 +225,7 @@ __device__ __forceinline__ void dev_fun(const CY &y, const CF &fix, const CR &rc
       a[r] = v;
     }
   }
-  if constexpr (SEG) {
+  if constexpr (SEG && M::TAIL == 0) {
     seg_gather<(U < 8 ? U : 8)>(0, M::NVAR, [&](int i) { return M::fv_ptr(i); },
                                 [&](int t) -> double { return M::fv_c(t); },
                                 [&](int t) -> double { return a[M::fv_r(t)]; },
@@ -214,9 +233,9 @@ __device__ __forceinline__ void dev_fun(const CY &y, const CF &fix, const CR &rc
   } else {
 #pragma unroll 1
     for (int i = 0; i < M::NVAR; ++i)
-      vdot[i] = gather_fma<U>(M::fv_ptr(i), M::fv_ptr(i + 1), 0.0,
-                              [&](int t) -> double { return M::fv_c(t); },
-                              [&](int t) -> double { return a[M::fv_r(t)]; });
+      vdot[i] = gather_sum<M, U>(M::fv_ptr(i), M::fv_ptr(i + 1), M::fv_ptr(i + 1), 0.0,
+                                 [&](int t) -> double { return M::fv_c(t); },
+                                 [&](int t) -> double { return a[M::fv_r(t)]; });
   }
 }
 
@@ -262,7 +281,7 @@ template <class M, int U = 1, bool SEG = false, class CY, class CF, class CR, cl
 __device__ void dev_jac(const CY &y, const CF &fix, const CR &rct, CB b, CO out, double sign,
                         double diag) {
   dev_partials<M, U>(y, fix, rct, b);
-  if constexpr (SEG) {
+  if constexpr (SEG && M::TAIL == 0) {
     seg_gather<(U < 8 ? U : 8)>(0, M::LU_NZ, [&](int k) { return M::jv_ptr(k); },
                                 [&](int t) -> double { return M::jv_c(t); },
                                 [&](int t) -> double { return b[M::jv_b(t)]; },
@@ -270,9 +289,9 @@ __device__ void dev_jac(const CY &y, const CF &fix, const CR &rct, CB b, CO out,
   } else {
 #pragma unroll 1
     for (int k = 0; k < M::LU_NZ; ++k) {
-      double acc = gather_fma<U>(M::jv_ptr(k), M::jv_ptr(k + 1), 0.0,
-                                 [&](int t) -> double { return M::jv_c(t); },
-                                 [&](int t) -> double { return b[M::jv_b(t)]; });
+      double acc = gather_sum<M, U>(M::jv_ptr(k), M::jv_ptr(k + 1), M::jv_ptr(k + 1), 0.0,
+                                    [&](int t) -> double { return M::jv_c(t); },
+                                    [&](int t) -> double { return b[M::jv_b(t)]; });
       out[k] = sign * acc;
     }
   }
@@ -347,9 +366,9 @@ __device__ int dev_jac_decomp(const CY &y, const CF &fix, const CR &rct, CB b, C
                               double diag) {
   dev_partials<M, U>(y, fix, rct, b);
   auto ghimj = [&](int q) -> double {
-    return sign * gather_fma<U>(M::jv_ptr(q), M::jv_ptr(q + 1), 0.0,
-                                [&](int t) -> double { return M::jv_c(t); },
-                                [&](int t) -> double { return b[M::jv_b(t)]; });
+    return sign * gather_sum<M, U>(M::jv_ptr(q), M::jv_ptr(q + 1), M::jv_ptr(q + 1), 0.0,
+                                   [&](int t) -> double { return M::jv_c(t); },
+                                   [&](int t) -> double { return b[M::jv_b(t)]; });
   };
   int ier = 0;
   int q = 0;
@@ -370,9 +389,9 @@ __device__ int dev_jac_decomp(const CY &y, const CF &fix, const CR &rct, CB b, C
         }
       }
       const double g = q == kd ? gd : ghimj(q);
-      double acc = gather_fma<U>(M::cr_ptr(q), M::cr_ptr(q + 1), g,
-                                 [&](int t) -> double { return -(double)lu[M::cr_l(t)]; },
-                                 [&](int t) -> double { return lu[M::cr_u(t)]; });
+      double acc = gather_sum<M, U>(M::cr_ptr(q), M::cr_hd(q), M::cr_ptr(q + 1), g,
+                                    [&](int t) -> double { return -(double)lu[M::cr_l(t)]; },
+                                    [&](int t) -> double { return lu[M::cr_u(t)]; });
       if (dv >= 0) acc = acc / lu[dv];
       lu[q] = acc;
     }
@@ -443,7 +462,7 @@ __device__ int dev_decomp_crout(CL lu) {
 // KppSolve in place: unit-lower forward then upper backward substitution.
 template <class M, int U = 1, bool SEG = false, class CL, class CX>
 __device__ void dev_solve(const CL &lu, CX x) {
-  if constexpr (SEG) {
+  if constexpr (SEG && M::TAIL == 0) {
     // forward: batches of rows that do not read each other; backward: the
     // numerators of a batch, then their divisions by the pivots
 #pragma unroll 1
@@ -473,14 +492,23 @@ __device__ void dev_solve(const CL &lu, CX x) {
   for (int i = 0; i < M::NVAR; ++i) {
     int k0 = M::lu_crow(i), k1 = M::lu_diag(i);
     if (k0 == k1) continue;
-    x[i] = gather_fma<U>(k0, k1, (double)x[i], [&](int k) -> double { return -(double)lu[k]; },
-                         [&](int k) -> double { return x[M::lu_icol(k)]; });
+    x[i] = gather_sum<M, U>(k0, M::fw_hd(i), k1, (double)x[i],
+                            [&](int k) -> double { return -(double)lu[k]; },
+                            [&](int k) -> double { return x[M::lu_icol(k)]; });
   }
 #pragma unroll 1
   for (int i = M::NVAR - 1; i >= 0; --i) {
     int kd = M::lu_diag(i), k1 = M::lu_crow(i + 1);
-    double acc = gather_fma<U>(kd + 1, k1, (double)x[i], [&](int k) -> double { return -(double)lu[k]; },
-                               [&](int k) -> double { return x[M::lu_icol(k)]; });
+    double acc;
+    if constexpr (M::TAIL == 0) {
+      acc = gather_fma<U>(kd + 1, k1, (double)x[i], [&](int k) -> double { return -(double)lu[k]; },
+                          [&](int k) -> double { return x[M::lu_icol(k)]; });
+    } else {  // descending columns, term t of the row at k1 - 1 - t
+      const int n = k1 - kd - 1;
+      acc = gather_sum<M, U>(0, i < M::NVAR - M::TAIL ? n : 0, n, (double)x[i],
+                             [&](int t) -> double { return -(double)lu[k1 - 1 - t]; },
+                             [&](int t) -> double { return x[M::lu_icol(k1 - 1 - t)]; });
+    }
     x[i] = acc / (double)lu[kd];
   }
 }
@@ -527,6 +555,19 @@ __device__ __forceinline__ void lc_wr(const LcLane &c, unsigned d, double v) {
 // loads and LDS instructions are not ordered with each other).
 __device__ __forceinline__ void lc_fence() { __builtin_amdgcn_s_waitcnt(0xc07f); }
 
+// Before the batch at term n of a sum (batches end at multiples of kChunk):
+// at a chunk's end the chunk's value moves into the sum and acc starts anew.
+template <class M>
+__device__ __forceinline__ void lc_chunk(int n, bool &chunks, double &sum, double &acc) {
+  if constexpr (M::TAIL > 0) {
+    if (n > 0 && n % kChunk == 0) {
+      sum = chunks ? sum + acc : acc;
+      chunks = true;
+      acc = 0.0;
+    }
+  }
+}
+
 // One batch of R terms of acc = fma(c(t), v(t), acc): a record of R bytes
 // (v's operand).  Returns the next record's word.
 template <int CS, int R, class DW, class FC, class FV>
@@ -548,18 +589,25 @@ __device__ __forceinline__ int lc_batch1(DW dw, int dp, const LcLane &c, int t, 
 }
 
 // acc = 0; acc = fma(c(t), v(t), acc) over [t, t1) in batches of 16 while
-// 16 remain, then of 8, 4, 2, 1 (the sizes the schedule assumes).
-template <int CS, class DW, class FC, class FV>
+// 16 remain, then of 8, 4, 2, 1 (the sizes the schedule assumes); with a tail
+// (M::TAIL) in chunks of kChunk terms as gather_sum adds them.
+template <class M, int CS, class DW, class FC, class FV>
 __device__ __forceinline__ double lc_sum1(DW dw, int &dp, const LcLane &c, int t, const int t1,
                                           FC cm, FV vm) {
-  double acc = 0.0;
+  double acc = 0.0, sum = 0.0;
+  const int t0 = t;
+  bool chunks = false;
 #pragma unroll 1
-  for (; t + 16 <= t1; t += 16) dp = lc_batch1<CS, 16>(dw, dp, c, t, acc, cm, vm);
+  for (; t + 16 <= t1; t += 16) {
+    lc_chunk<M>(t - t0, chunks, sum, acc);
+    dp = lc_batch1<CS, 16>(dw, dp, c, t, acc, cm, vm);
+  }
+  if (t < t1) lc_chunk<M>(t - t0, chunks, sum, acc);
   if (t + 8 <= t1) { dp = lc_batch1<CS, 8>(dw, dp, c, t, acc, cm, vm); t += 8; }
   if (t + 4 <= t1) { dp = lc_batch1<CS, 4>(dw, dp, c, t, acc, cm, vm); t += 4; }
   if (t + 2 <= t1) { dp = lc_batch1<CS, 2>(dw, dp, c, t, acc, cm, vm); t += 2; }
   if (t < t1) dp = lc_batch1<CS, 1>(dw, dp, c, t, acc, cm, vm);
-  return acc;
+  return chunks ? sum + acc : acc;
 }
 
 // Extra operands and result of a two-operand sum (its first record's header
@@ -610,12 +658,15 @@ __device__ __forceinline__ int lc_batch2(DW dw, int dp, const LcLane &c, int t, 
 }
 
 // acc = (h.init_x0 ? x0 : h.init); acc = fma(-a(t), b(t), acc) over
-// [t, t1), batches as in lc_sum1 (the first carries the header).
-template <int CS, class DW, class FX0, class FX2, class FA, class FB>
-__device__ __forceinline__ double lc_sum2(DW dw, int &dp, const LcLane &c, int t, const int t1,
-                                          LcHead &h, FX0 x0m, FX2 x2m, FA am, FB bm) {
-  double acc = 0.0;
-  const int n = t1 - t;
+// [t, t1), batches as in lc_sum1 (the first carries the header): the terms
+// before th in chunks as gather_sum adds them, then those from th on.
+template <class M, int CS, class DW, class FX0, class FX2, class FA, class FB>
+__device__ __forceinline__ double lc_sum2(DW dw, int &dp, const LcLane &c, int t, const int th,
+                                          const int t1, LcHead &h, FX0 x0m, FX2 x2m, FA am, FB bm) {
+  double acc = 0.0, sum = 0.0;
+  const int t0 = t;
+  bool chunks = false;
+  const int n = th - t;
   if (n >= 16) { dp = lc_batch2<CS, 16, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 16; }
   else if (n >= 8) { dp = lc_batch2<CS, 8, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 8; }
   else if (n >= 4) { dp = lc_batch2<CS, 4, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 4; }
@@ -623,12 +674,21 @@ __device__ __forceinline__ double lc_sum2(DW dw, int &dp, const LcLane &c, int t
   else if (n == 1) { dp = lc_batch2<CS, 1, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 1; }
   else dp = lc_batch2<CS, 0, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm);
 #pragma unroll 1
-  for (; t + 16 <= t1; t += 16)
-    dp = lc_batch2<CS, 16, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm);
-  if (t + 8 <= t1) { dp = lc_batch2<CS, 8, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 8; }
-  if (t + 4 <= t1) { dp = lc_batch2<CS, 4, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 4; }
-  if (t + 2 <= t1) { dp = lc_batch2<CS, 2, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 2; }
-  if (t < t1) dp = lc_batch2<CS, 1, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm);
+  for (int part = 0; part < 2; ++part) {  // before th, then from th on
+    const int te = part ? t1 : th;
+#pragma unroll 1
+    for (; t + 16 <= te; t += 16) {
+      if (!part) lc_chunk<M>(t - t0, chunks, sum, acc);
+      dp = lc_batch2<CS, 16, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm);
+    }
+    if (!part && t < te) lc_chunk<M>(t - t0, chunks, sum, acc);
+    if (t + 8 <= te) { dp = lc_batch2<CS, 8, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 8; }
+    if (t + 4 <= te) { dp = lc_batch2<CS, 4, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 4; }
+    if (t + 2 <= te) { dp = lc_batch2<CS, 2, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 2; }
+    if (t < te) { dp = lc_batch2<CS, 1, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 1; }
+    if (!part && chunks) acc = sum + acc;
+    if (th == t1) break;
+  }
   return acc;
 }
 
@@ -640,7 +700,7 @@ __device__ __forceinline__ int dev_jac_decomp_c(const CY &y, const CF &fix, cons
   auto dw = [&](int i) { return M::lc_lu(CS, i); };
   int dp = 0;
   auto ghimj = [&](int q) -> double {
-    return sign * lc_sum1<CS>(dw, dp, c, M::jv_ptr(q), M::jv_ptr(q + 1),
+    return sign * lc_sum1<M, CS>(dw, dp, c, M::jv_ptr(q), M::jv_ptr(q + 1),
                           [&](int t) -> double { return M::jv_c(t); },
                           [&](int t) { return b[M::jv_b(t)]; });
   };
@@ -657,7 +717,8 @@ __device__ __forceinline__ int dev_jac_decomp_c(const CY &y, const CF &fix, cons
       const double g = q == kd ? gd : ghimj(q);
       const int dv = M::cr_div(q);
       LcHead h{dv >= 0, false, false, g, 0.0, 0.0, 0u};
-      double acc = lc_sum2<CS>(dw, dp, c, M::cr_ptr(q), M::cr_ptr(q + 1), h,
+      const int th = M::TAIL > 0 ? M::cr_hd(q) : M::cr_ptr(q + 1);
+      double acc = lc_sum2<M, CS>(dw, dp, c, M::cr_ptr(q), th, M::cr_ptr(q + 1), h,
                            [&]() { return lu[dv]; }, [&]() { return lu[0]; },
                            [&](int t) { return lu[M::cr_l(t)]; },
                            [&](int t) { return lu[M::cr_u(t)]; });
@@ -679,7 +740,8 @@ __device__ __forceinline__ void dev_solve_c(const CL &lu, CX x, const LcLane &c)
     const int k0 = M::lu_crow(i), k1 = M::lu_diag(i);
     if (k0 == k1) continue;
     LcHead h{true, false, true, 0.0, 0.0, 0.0, 0u};
-    const double acc = lc_sum2<CS>(dw, dp, c, k0, k1, h, [&]() { return x[i]; },
+    const double acc = lc_sum2<M, CS>(dw, dp, c, k0, M::TAIL > 0 ? M::fw_hd(i) : k1, k1, h,
+                               [&]() { return x[i]; },
                                [&]() { return x[i]; }, [&](int k) { return lu[k]; },
                                [&](int k) { return x[M::lu_icol(k)]; });
     x[i] = acc;
@@ -689,9 +751,12 @@ __device__ __forceinline__ void dev_solve_c(const CL &lu, CX x, const LcLane &c)
   for (int i = M::NVAR - 1; i >= 0; --i) {
     const int kd = M::lu_diag(i), k1 = M::lu_crow(i + 1);
     LcHead h{true, true, true, 0.0, 0.0, 0.0, 0u};
-    double acc = lc_sum2<CS>(dw, dp, c, kd + 1, k1, h, [&]() { return x[i]; },
-                         [&]() { return lu[kd]; }, [&](int k) { return lu[k]; },
-                         [&](int k) { return x[M::lu_icol(k)]; });
+    const int n = k1 - kd - 1;  // with a tail descending columns, as in dev_solve
+    auto at = [&](int t) { return M::TAIL > 0 ? k1 - 1 - t : kd + 1 + t; };
+    double acc = lc_sum2<M, CS>(dw, dp, c, 0, M::TAIL > 0 && i >= M::NVAR - M::TAIL ? 0 : n, n, h,
+                                [&]() { return x[i]; }, [&]() { return lu[kd]; },
+                                [&](int t) { return lu[at(t)]; },
+                                [&](int t) { return x[M::lu_icol(at(t))]; });
     acc = acc / h.x2v;
     x[i] = acc;
     lc_wr<CS>(c, h.res, acc);
@@ -952,7 +1017,7 @@ __device__ __forceinline__ bool lane_attempt(const IntegrateArgs &a, const Slot 
   bool singular = true;
   while (singular) {
     int ising;
-    if constexpr (SEG) {
+    if constexpr (SEG && M::TAIL == 0) {
       dev_jac<M, U, SEG>(Yc, Yc, rct, Ascr, LU, -1.0, 1.0 / (dir * S.H * kRosGamma1));
       ising = dev_decomp_crout<M, U, SEG>(LU);
     } else if constexpr (CS > 0) {
@@ -1019,6 +1084,24 @@ __device__ __forceinline__ bool lane_attempt(const IntegrateArgs &a, const Slot 
     double sc = P.vectol ? a.atol[i] + a.rtol[i] * ymax : a.atol[0] + a.rtol[0] * ymax;
     qq = ye / sc;
   };
+  if constexpr (M::TAIL > 0) {
+    // species l, l + 64, ... summed for each l, then the sums in l order (the
+    // cell-per-wave solver's lanes)
+#pragma unroll 1
+    for (int l = 0; l < 64; ++l) {
+      constexpr int KS = (M::NVAR + 63) / 64;
+      double v[KS], qq[KS], part = 0.0;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) err_term(min(l + 64 * k, N - 1), v[k], qq[k]);
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (l + 64 * k < N) {
+          Ynew[l + 64 * k] = v[k];
+          part = fma(qq[k], qq[k], part);
+        }
+      err += part;
+    }
+  } else
   {
     int i = 0;
     if constexpr (VB > 1) {
@@ -1421,7 +1504,7 @@ const void *persist_kernel_variant(int qset, int variant) {
     case 4: return persist_kernel<16, 4, false>(qset);
     case 5: return persist_kernel<16, 4, true>(qset);
     case 6: return persist_kernel<8, 5, false>(qset);
-    case PERSIST_WAVE_VARIANT: return wave_kernel(qset);
+    case PERSIST_WAVE_VARIANT: return wave_kernel(qset).fn;
     case 8: return persist_kernel<16, 4, false, 16>(qset);
     case 9: return persist_kernel<16, 2, false, 32>(qset);
   }
@@ -1462,23 +1545,42 @@ int64_t persist_resident_waves(int qset, int variant, int wpb) {
   if (variant == PERSIST_WAVE_VARIANT && wpb != 1) return 0;  // its workgroup is one wave
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   const int cs = persist_variant_cache(variant);
-  const size_t lds = cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
+  size_t lds = cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
+  if (variant == PERSIST_WAVE_VARIANT) {
+    wpb = wave_kernel(qset).max_wpb;
+    lds = wave_kernel(qset).lds(wpb);
+  }
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 64 * wpb, lds) != hipSuccess) return 0;
   return (int64_t)ncu * (per > 0 ? per : 1) * wpb;
 }
+// Cell-per-wave launches up to this many waves take a workgroup for each wave:
+// two one-wave workgroups fit a CU, so 256 CUs still hold them all at once,
+// and fewer waves share a CU's LDS than in workgroups of three.
+constexpr int64_t kWaveSpread = 512;
+
 // nwaves waves in workgroups of wpb waves; counter null: one cell per lane
 // (nwaves*64 >= cells), else work stealing from *counter (zeroed here by a
 // kernel, so the launch pair can be captured in a graph).
-int launch_persist(int qset, int variant, int wpb, const PersistArgs &pa, int64_t nwaves,
+int launch_persist(int qset, int variant, int wpb, const PersistArgs &args0, int64_t nwaves,
                    hipStream_t s) {
+  PersistArgs pa = args0;
+  pa.nwaves = nwaves;
   const void *k = persist_kernel_variant(qset, variant);
   if (!k || nwaves <= 0 || wpb < 1 || wpb > 4 || nwaves % wpb) return -1;
   if (variant == PERSIST_WAVE_VARIANT && wpb != 1) return -1;
   if (pa.counter) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, pa.counter);
   void *args[] = {(void *)&pa};
   const int cs = persist_variant_cache(variant);
-  const size_t lds = cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
-  return hipLaunchKernel(k, dim3((unsigned)(nwaves / wpb)), dim3(64 * wpb), args, lds, s) ==
+  size_t lds = cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
+  int64_t blocks = nwaves / wpb;
+  if (variant == PERSIST_WAVE_VARIANT) {
+    // few waves: a workgroup (and so a CU's LDS) for each
+    const WaveKernel w = wave_kernel(qset);
+    wpb = nwaves > kWaveSpread ? w.max_wpb : 1;
+    lds = w.lds(wpb);
+    blocks = (nwaves + wpb - 1) / wpb;
+  }
+  return hipLaunchKernel(k, dim3((unsigned)blocks), dim3(64 * wpb), args, lds, s) ==
                  hipSuccess
              ? 0 : -1;
 }

@@ -1,15 +1,15 @@
 // Rodas3 solve with one wavefront per cell.  The lane-per-cell solvers
 // (rosenbrock.hip) keep each cell's state in HBM and stream ~1.3 MB per
-// Rodas3 attempt; here the cell's LU, solve vector and state live in LDS
-// (fullchem: 51 KB, three cells per CU) and the 64 lanes share its sums.
-// The reaction products, Jacobian partials, rate constants, Fcn0 and the
-// stage vectors sit in the wave's global scratch (about 37 KB, L2-resident).
-// Every sum -- a Vdot row, a Jacobian entry, an LU position (row-Crout
-// form), a substitution row -- is computed by one lane, term by term in the
-// same order and with the same operations as the lane-per-cell solvers, so
-// the results are bit-identical to theirs.  The mechanism's wave programs
-// (gen/mech_<name>.h, built by mechgen/wave_sched.py) say which lane
-// computes which chunk of which sum in which round.
+// Rodas3 attempt; here the cell's LU, solve vector and state live in LDS and
+// the 64 lanes share its sums.  Every chunk of a sum -- a Vdot row, a Jacobian
+// entry, an LU position (row-Crout form), a substitution row -- is computed by
+// one lane, term by term in the same order and with the same operations as
+// the lane-per-cell solvers, so the results are bit-identical to theirs.
+// A mechanism with a tail block (M::TAIL > 0, fullchem) runs the cell programs
+// of mechgen/cell_sched.py (cell_solver.h); a small one (Hg, carbon) the wave
+// programs of mechgen/wave_sched.py below, with its reaction products,
+// partials, rate constants, Fcn0 and stage vectors in the wave's global
+// scratch.
 //
 // Algorithm: that of lane_attempt in rosenbrock.hip (ros_Integrator,
 // KPP/fullchem/gckpp_Integrator.F90:578-786, Rodas3 :2239-2303).
@@ -344,18 +344,9 @@ __device__ __forceinline__ void wave_zero_slots(const WaveCell<M> &c) {
   }
 }
 
-template <class M>
-__device__ void wave_begin(const IntegrateArgs &a, const WaveCell<M> &c, int64_t cell, bool cold,
-                           WaveState &S) {
-  double *sh = c.sh;
-  double *rct = c.rct();
-  wave_sync_global();
-#pragma unroll 1
-  for (int s = c.lane; s < M::NSPEC; s += 64) sh[M::WV_Y0 + s] = a.conc[(int64_t)s * a.cstride + cell];
-#pragma unroll 1
-  for (int r = c.lane; r < M::NREACT; r += 64) rct[r] = a.rconst[(int64_t)r * a.rstride + cell];
-  wave_zero_slots(c);
-  wave_sync_global();
+// The integrator state at the start of a cell's integration.
+__device__ __forceinline__ void state_begin(const IntegrateArgs &a, int64_t cell, bool cold,
+                                            WaveState &S) {
   const RosParams &P = a.prm;
   const double hs = (a.hstart && !cold) ? a.hstart[cell] : 0.0;
   double Hstart = P.Hstart_default;
@@ -370,6 +361,19 @@ __device__ void wave_begin(const IntegrateArgs &a, const WaveCell<M> &c, int64_t
   S.ierr = 1;
   S.rejLast = S.rejMore = false;
   S.newStep = true;
+}
+
+template <class M>
+__device__ void wave_begin(const IntegrateArgs &a, const WaveCell<M> &c, int64_t cell) {
+  double *sh = c.sh;
+  double *rct = c.rct();
+  wave_sync_global();
+#pragma unroll 1
+  for (int s = c.lane; s < M::NSPEC; s += 64) sh[M::WV_Y0 + s] = a.conc[(int64_t)s * a.cstride + cell];
+#pragma unroll 1
+  for (int r = c.lane; r < M::NREACT; r += 64) rct[r] = a.rconst[(int64_t)r * a.rstride + cell];
+  wave_zero_slots(c);
+  wave_sync_global();
 }
 
 // One Rodas3 attempt of the wave's cell (lane_attempt's algorithm); true
@@ -577,25 +581,13 @@ __device__ void wave_euler(const IntegrateArgs &a, const WaveCell<M> &c, WaveSta
   S.ierr = 1;
 }
 
-// Continues a cell the lane kernel handed off at a step boundary (entry idx
-// of the hand-off list; see Handoff): Y of the variable species and the
-// integrator state from the list, the fixed species and the rate constants
-// from conc and rconst as wave_begin reads them.
-template <class M>
-__device__ void wave_resume(const IntegrateArgs &a, const Handoff &ho, const WaveCell<M> &c,
-                            int64_t cell, int64_t idx, WaveState &S) {
-  double *sh = c.sh;
-  double *rct = c.rct();
+// The state of a cell the lane kernel handed off at a step boundary (entry
+// idx of the hand-off list; see Handoff).  Y of the variable species is in
+// the list too; the fixed species and the rate constants come from conc and
+// rconst as at the start of a cell.
+__device__ __forceinline__ void state_resume(const Handoff &ho, int64_t idx, WaveState &S) {
   const double *r = ho.rec + idx;
   const int64_t cap = ho.cap;
-  wave_sync_global();
-#pragma unroll 1
-  for (int s = c.lane; s < M::NSPEC; s += 64)
-    sh[M::WV_Y0 + s] = s < M::NVAR ? r[(HO_FIELDS + s) * cap] : a.conc[(int64_t)s * a.cstride + cell];
-#pragma unroll 1
-  for (int k = c.lane; k < M::NREACT; k += 64) rct[k] = a.rconst[(int64_t)k * a.rstride + cell];
-  wave_zero_slots(c);
-  wave_sync_global();
   S.T = r[0];
   S.H = r[cap];
   S.Hnew = S.H;
@@ -610,8 +602,24 @@ __device__ void wave_resume(const IntegrateArgs &a, const Handoff &ho, const Wav
 }
 
 template <class M>
-__device__ void wave_finish(const IntegrateArgs &a, const WaveCell<M> &c, int64_t cell,
-                            const WaveState &S) {
+__device__ void wave_resume(const IntegrateArgs &a, const Handoff &ho, const WaveCell<M> &c,
+                            int64_t cell, int64_t idx) {
+  double *sh = c.sh;
+  double *rct = c.rct();
+  const double *r = ho.rec + idx;
+  const int64_t cap = ho.cap;
+  wave_sync_global();
+#pragma unroll 1
+  for (int s = c.lane; s < M::NSPEC; s += 64)
+    sh[M::WV_Y0 + s] = s < M::NVAR ? r[(HO_FIELDS + s) * cap] : a.conc[(int64_t)s * a.cstride + cell];
+#pragma unroll 1
+  for (int k = c.lane; k < M::NREACT; k += 64) rct[k] = a.rconst[(int64_t)k * a.rstride + cell];
+  wave_zero_slots(c);
+  wave_sync_global();
+}
+
+template <class M>
+__device__ void wave_finish(const IntegrateArgs &a, const WaveCell<M> &c, int64_t cell) {
   const double *sh = c.sh;
   const int nout = a.clip_out ? M::NSPEC : M::NVAR;
 #pragma unroll 1
@@ -620,7 +628,10 @@ __device__ void wave_finish(const IntegrateArgs &a, const WaveCell<M> &c, int64_
     if (a.clip_out) v = v > 0.0 ? v : 0.0;
     a.conc[(int64_t)s * a.cstride + cell] = v;
   }
-  const int k = c.lane;
+}
+
+__device__ __forceinline__ void state_finish(const IntegrateArgs &a, int k, int64_t cell,
+                                             const WaveState &S) {
   int stk = 0;  // S.st[k] without a lane-indexed (scratch) array access
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -636,6 +647,8 @@ __device__ void wave_finish(const IntegrateArgs &a, const WaveCell<M> &c, int64_
   }
 }
 
+#include "cell_solver.h"
+
 template <class M0, class M1, class M2, class Fn>
 __device__ __forceinline__ void on_queue_w(int q, Fn &&f) {
   if constexpr (!std::is_void_v<M2>) {
@@ -647,22 +660,54 @@ __device__ __forceinline__ void on_queue_w(int q, Fn &&f) {
   f((M0 *)nullptr);
 }
 
-template <class M> struct WvSh { static constexpr int v = M::WV_SH; };
-template <> struct WvSh<void> { static constexpr int v = 0; };
 template <class M> struct IsEulerW : std::false_type {};
 template <> struct IsEulerW<Traits_carbon> : std::true_type {};
+template <class M> struct HasCell : std::bool_constant<(M::TAIL > 0)> {};
+template <> struct HasCell<void> : std::false_type {};
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
-// One wave (= one workgroup) per resident slot; cells from the queues of
-// PersistArgs by work stealing (or one cell per wave when counter is null),
-// with the step-mode retry, clip and RSTATUS(3) write-back of k_persist.
+// LDS of a queue set's kernel: the coefficient table of the cell programs
+// (one for the workgroup's waves), then a block per wave, in doubles.
+template <class M, bool CELL = HasCell<M>::value> struct WvLds {
+  static constexpr int SH = CellProg<M>::SIZE, NCOEF = CellProg<M>::NCOEF, WPB = CellProg<M>::CELLS;
+};
+template <class M> struct WvLds<M, false> {
+  static constexpr int SH = M::WV_SH, NCOEF = 0, WPB = 1;
+};
+template <> struct WvLds<void, false> { static constexpr int SH = 0, NCOEF = 0, WPB = 1; };
+template <class M0, class M1, class M2> struct QueueLds {
+  static constexpr int SH = cmax(WvLds<M0>::SH, cmax(WvLds<M1>::SH, WvLds<M2>::SH));
+  static constexpr int NCOEF = WvLds<M0>::NCOEF, WPB = WvLds<M0>::WPB;
+  static_assert(!HasCell<M1>::value && !HasCell<M2>::value, "the first queue has the cell programs");
+};
+struct NoCell {};
+
+// A workgroup of one wave, or, with cell programs, of as many as its LDS
+// holds (they share the coefficient table); every wave works by itself, on
+// cells from the queues of PersistArgs by work stealing (or one cell per
+// wave when counter is null), with the step-mode retry, clip and RSTATUS(3)
+// write-back of k_persist.
 template <class M0, class M1, class M2>
-__global__ __launch_bounds__(64) void k_wave(PersistArgs pa) {
-  constexpr int SH = cmax(WvSh<M0>::v, cmax(WvSh<M1>::v, WvSh<M2>::v));
-  __shared__ double sh[SH];
-  const int lane = threadIdx.x;
-  const int64_t wave = blockIdx.x;
+__global__ __launch_bounds__((64 * QueueLds<M0, M1, M2>::WPB), 1) void k_wave(PersistArgs pa) {
+  using Lds = QueueLds<M0, M1, M2>;
+  constexpr bool CELL = HasCell<M0>::value;
+  extern __shared__ double wv_lds[];
+  const int lane = threadIdx.x & 63;
+  const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + wib;
+  double *const sh = wv_lds + Lds::NCOEF + wib * Lds::SH;
+  CellLds cl{};
+  std::conditional_t<CELL, CellState<std::conditional_t<CELL, M0, Traits_fullchem>>, NoCell> cs;
+  if constexpr (CELL) {
+    for (int i = threadIdx.x; i < Lds::NCOEF; i += blockDim.x) wv_lds[i] = CellProg<M0>::coef(i);
+    cl.coef = (unsigned)(uintptr_t)(lds_double *)wv_lds;
+    cl.base = cl.coef + 8u * (Lds::NCOEF + wib * Lds::SH);
+    cl.own = cl.base + 8u * lane;
+    cl.lane = lane;
+    __syncthreads();
+    if (wave >= pa.nwaves) return;
+  }
   double *g = pa.work + wave * (64 * pa.slot_fields);
   constexpr int NQ = std::is_void_v<M1> ? 1 : (std::is_void_v<M2> ? 2 : 3);
   int64_t total = pa.qend[NQ - 1];
@@ -674,6 +719,14 @@ __global__ __launch_bounds__(64) void k_wave(PersistArgs pa) {
   int q = 0;
   int64_t next_static = wave;
   WaveState S;
+  auto begin = [&](bool cold) {
+    on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
+      using M = std::remove_pointer_t<decltype(tag)>;
+      if constexpr (HasCell<M>::value) cell_begin<M>(pa.q[q], cl, cell, cs);
+      else wave_begin<M>(pa.q[q], WaveCell<M>{sh, g, lane}, cell);
+    });
+    state_begin(pa.q[q], cell, cold, S);
+  };
   for (;;) {
     if (cell < 0) {
       int64_t cidx;
@@ -683,7 +736,7 @@ __global__ __launch_bounds__(64) void k_wave(PersistArgs pa) {
         cidx = (int64_t)__builtin_amdgcn_readfirstlane(v);
       } else {
         cidx = next_static;
-        next_static += gridDim.x;
+        next_static += pa.nwaves;
       }
       if (cidx >= total) break;
       if (pa.ho.resume) {
@@ -691,9 +744,13 @@ __global__ __launch_bounds__(64) void k_wave(PersistArgs pa) {
         cell = pa.ho.cell[cidx];
         on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
           using M = std::remove_pointer_t<decltype(tag)>;
-          if constexpr (!IsEulerW<M>::value)
-            wave_resume<M>(pa.q[q], pa.ho, WaveCell<M>{sh, g, lane}, cell, cidx, S);
+          if constexpr (HasCell<M>::value) {
+            cell_resume<M>(pa.q[q], pa.ho, cl, cell, cidx, cs);
+          } else if constexpr (!IsEulerW<M>::value) {
+            wave_resume<M>(pa.q[q], pa.ho, WaveCell<M>{sh, g, lane}, cell, cidx);
+          }
         });
+        state_resume(pa.ho, cidx, S);
       } else {
         // queue of the cell: the number of queue ends at or below cidx (the
         // ends are nondecreasing).  Written as a sum of compares: the
@@ -706,22 +763,20 @@ __global__ __launch_bounds__(64) void k_wave(PersistArgs pa) {
         cell = cidx - (q ? pa.qend[q - 1] : 0);
         if (pa.q[q].order) cell = pa.q[q].order[cell];
         S.tries = 0;
-        on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
-          using M = std::remove_pointer_t<decltype(tag)>;
-          wave_begin<M>(pa.q[q], WaveCell<M>{sh, g, lane}, cell, false, S);
-        });
+        begin(false);
       }
     }
     bool done = false;
     const int nstp0 = S.st[2];
     on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
       using M = std::remove_pointer_t<decltype(tag)>;
-      const WaveCell<M> c{sh, g, lane};
-      if constexpr (IsEulerW<M>::value) {
-        wave_euler<M>(pa.q[q], c, S);
+      if constexpr (HasCell<M>::value) {
+        done = cell_attempt<M>(pa.q[q], cl, cell, S, cs);
+      } else if constexpr (IsEulerW<M>::value) {
+        wave_euler<M>(pa.q[q], WaveCell<M>{sh, g, lane}, S);
         done = true;
       } else {
-        done = wave_attempt<M>(pa.q[q], c, cell, S);
+        done = wave_attempt<M>(pa.q[q], WaveCell<M>{sh, g, lane}, cell, S);
       }
     });
     if (pa.ho.resume && lane == 0 && S.st[2] != nstp0)
@@ -729,21 +784,26 @@ __global__ __launch_bounds__(64) void k_wave(PersistArgs pa) {
     if (done) {
       const IntegrateArgs &a = pa.q[q];
       if (S.ierr < 0 && a.retry && S.tries == 0) {
-        on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
-          using M = std::remove_pointer_t<decltype(tag)>;
-          wave_begin<M>(a, WaveCell<M>{sh, g, lane}, cell, true, S);
-        });
+        begin(true);
         S.tries = 1;
       } else {
         on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
           using M = std::remove_pointer_t<decltype(tag)>;
-          wave_finish<M>(a, WaveCell<M>{sh, g, lane}, cell, S);
+          if constexpr (HasCell<M>::value) cell_finish<M>(a, cl, cell, cs);
+          else wave_finish<M>(a, WaveCell<M>{sh, g, lane}, cell);
         });
+        state_finish(a, lane, cell, S);
         wave_sync();
         cell = -1;
       }
     }
   }
+}
+
+template <class M0, class M1, class M2>
+WaveKernel wave_of() {
+  using Lds = QueueLds<M0, M1, M2>;
+  return WaveKernel{(const void *)k_wave<M0, M1, M2>, Lds::WPB, Lds::NCOEF, Lds::SH};
 }
 
 }  // namespace
@@ -763,16 +823,15 @@ int64_t wave_scratch_fields(int qset) {
   return (g + 63) / 64;
 }
 
-// The cell-per-wave kernel for a queue set (PQ_*), launched with 64 threads
-// per workgroup.
-const void *wave_kernel(int qset) {
+// The cell-per-wave kernel for a queue set (PQ_*).
+WaveKernel wave_kernel(int qset) {
   switch (qset) {
-    case PQ_FULLCHEM: return (const void *)k_wave<Traits_fullchem, void, void>;
-    case PQ_HG: return (const void *)k_wave<Traits_Hg, void, void>;
-    case PQ_CARBON: return (const void *)k_wave<Traits_carbon, void, void>;
-    case PQ_MIXED: return (const void *)k_wave<Traits_fullchem, Traits_Hg, Traits_carbon>;
+    case PQ_FULLCHEM: return wave_of<Traits_fullchem, void, void>();
+    case PQ_HG: return wave_of<Traits_Hg, void, void>();
+    case PQ_CARBON: return wave_of<Traits_carbon, void, void>();
+    case PQ_MIXED: return wave_of<Traits_fullchem, Traits_Hg, Traits_carbon>();
   }
-  return nullptr;
+  return WaveKernel{nullptr, 1, 0, 0};
 }
 
 }  // namespace gckpp

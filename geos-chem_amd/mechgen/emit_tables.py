@@ -29,6 +29,7 @@ import sys
 from pathlib import Path
 
 sys.path.insert(0, str(Path(__file__).resolve().parent))
+import cell_sched  # noqa: E402
 import lane_cache  # noqa: E402
 import wave_sched  # noqa: E402
 
@@ -105,9 +106,16 @@ def build_tables(m):
                 if kk is None:
                     raise ValueError("Jacobian entry (%d,%d) outside LU pattern" % (i, s))
                 jterms[kk].append((b, c))
+    # (with cell programs, the batch a partial is made in comes first)
+    made = [0] * len(pt_r)
+    if nz and cell_sched.tail_size(m):
+        rslot, _ = cell_sched.reaction_rows(m)
+        batch, _ = cell_sched.partial_batches(m)
+        for b, ri in enumerate(pt_r):
+            made[b] = batch[(rslot[ri] // cell_sched.LANES, b - pt_r.index(ri))]
     jv_ptr, jv_b, jv_c = [0], [], []
     for k in range(nz):
-        for b, c in sorted(jterms[k]):
+        for b, c in sorted(jterms[k], key=lambda x: (made[x[0]], x)):
             jv_b.append(b)
             jv_c.append(c)
         jv_ptr.append(len(jv_b))
@@ -152,6 +160,14 @@ def build_tables(m):
             cr_ptr.append(len(cr_l))
             cr_div.append(diag[c] if c < k else -1)
     assert len(cr_l) == len(lp_dst)
+    # where a sum's terms from in front of the tail block end (cell_sched):
+    # cr_hd per LU position, fw_hd per row of the forward substitution
+    tail = cell_sched.tail_size(m) if nz else 0
+    s0 = nvar - tail
+    cr_hd = [cr_ptr[q] + sum(1 for x in range(cr_ptr[q], cr_ptr[q + 1]) if lu_icol[cr_l[x]] < s0)
+             for q in range(nz)]
+    fw_hd = [crow[k] + sum(1 for q in range(crow[k], diag[k]) if lu_icol[q] < s0)
+             for k in range(nvar if nz else 0)]
     # flat segmented forms for latency-batched execution: each segment's
     # first term carries its initial value with l index LU_NONZERO, the
     # solver's constant entry -lu[LU_NONZERO] = 1 (see the persistent slot)
@@ -195,13 +211,34 @@ def build_tables(m):
         sb_sp, sb_l, sb_x, sb_batch = solve_tables(list(range(nvar - 1, -1, -1)), False)
     else:
         sf_sp = sf_l = sf_x = sf_batch = sb_sp = sb_l = sb_x = sb_batch = []
-    return dict(cu_row=cu_row, cu_sp=cu_sp, cu_q=cu_q, cu_l=cu_l, cu_u=cu_u,
+    return dict(cr_hd=cr_hd, fw_hd=fw_hd, cu_row=cu_row, cu_sp=cu_sp, cu_q=cu_q, cu_l=cu_l, cu_u=cu_u,
                 sf_sp=sf_sp, sf_l=sf_l, sf_x=sf_x, sf_batch=sf_batch,
                 sb_sp=sb_sp, sb_l=sb_l, sb_x=sb_x, sb_batch=sb_batch,
                 rx_s=rx_s, fv_ptr=fv_ptr, fv_r=fv_r, fv_c=fv_c, pt_r=pt_r, pt_m=pt_m,
                 pt_s=pt_s, jv_ptr=jv_ptr, jv_b=jv_b, jv_c=jv_c, le_kk=le_kk, le_dj=le_dj,
                 le_p0=le_p0, le_p1=le_p1, le_row=le_row, lp_dst=lp_dst, lp_src=lp_src,
                 row_e0=row_e0, cr_ptr=cr_ptr, cr_l=cr_l, cr_u=cr_u, cr_div=cr_div)
+
+
+def cell_text(name, m, t, cell):
+    """The header of a mechanism's cell programs (cell_sched.py)."""
+    L = cell["layout"]
+    code, words, _ = cell_sched.emit_code(m, t, cell)
+    rx = [0] * cell["na"]
+    for r, p in enumerate(cell["slot"]):
+        rx[p] = r
+    out = ["/* Generated by geos-chem_amd/mechgen/emit_tables.py from mech/%s.json"
+           " -- do not edit. */" % name, "#pragma once", "", "namespace cell_%s {" % name,
+           "constexpr int TAIL = %d, ROWS = %d, NREACT = %d, NCOEF = %d, SIZE = %d, CELLS = %d;"
+           % (cell["tail"], len(cell["rows"]), m["nreact"], len(cell["coef"]), L["SIZE"],
+              cell_sched.KCELLS),
+           "constexpr int X0 = %d, ZERO = %d, ONE = %d, NEG = %d, SINK = %d;"
+           % (L["X"], L["ZERO"], L["ONE"], L["NEG"], L["SINK"]),
+           arr("int", "rx", rx), arr("double", "coef", cell["coef"], per_line=6, fmt=dfmt)]
+    for k, v in words.items():
+        out.append(arr("unsigned", k, v, align=16))
+    out += [code, "}  // namespace cell_%s" % name, ""]
+    return "\n".join(out)
 
 
 def emit(name):
@@ -219,7 +256,7 @@ def emit(name):
            % (max(0, len(t["sf_batch"]) - 1), max(0, len(t["sb_batch"]) - 1)), ""]
     ints = ["rx_s", "fv_ptr", "fv_r", "pt_r", "pt_s", "jv_ptr", "jv_b", "le_kk", "le_dj",
             "le_p0", "le_p1", "le_row", "lp_dst", "lp_src", "row_e0", "cr_ptr", "cr_l", "cr_u",
-            "cr_div", "cu_row", "cu_sp", "cu_q", "cu_l", "cu_u", "sf_sp", "sf_l", "sf_x",
+            "cr_div", "cr_hd", "fw_hd", "cu_row", "cu_sp", "cu_q", "cu_l", "cu_u", "sf_sp", "sf_l", "sf_x",
             "sf_batch", "sb_sp", "sb_l", "sb_x", "sb_batch"]
     for k in ints:
         out.append(arr("int", k, t[k]))
@@ -258,10 +295,14 @@ def emit(name):
         lw, sw = lane_cache.build(m, t, S)
         out.append(arr("unsigned", "lc%d_lu" % S, lw + [0] * 16))
         out.append(arr("unsigned", "lc%d_sv" % S, sw + [0] * 16))
+    out.append("constexpr int TAIL = %d;" % cell_sched.tail_size(m))
     out.append("}  // namespace mech_%s" % name)
     gen = HERE.parent / "csrc" / "gen"
     gen.mkdir(exist_ok=True)
     (gen / ("mech_%s.h" % name)).write_text("\n".join(out) + "\n")
+    cell = cell_sched.build(m, t)
+    if cell:
+        (gen / ("cell_%s.h" % name)).write_text(cell_text(name, m, t, cell))
     print("%s: NFV=%d NPART=%d NJV=%d NLE=%d NLP=%d" % (name, len(t["fv_r"]), len(t["pt_r"]),
                                                        len(t["jv_b"]), len(t["le_kk"]), len(t["lp_dst"])))
 

@@ -46,6 +46,8 @@ before the schedule reads it), so a section can be restarted at any time
 (singular-matrix retries).  Every result also goes to the slot block (LU
 entries and x values are read after the section).
 """
+import cell_sched
+
 SLOTS = (16, 32)   # cache sizes the kernels are built for
 MEM, HIT, FILL, NONE = 0, 1, 2, 3
 INF = 1 << 60
@@ -88,7 +90,10 @@ def lu_events(m, t):
             if q != kd:
                 ghimj(q)
             dv = t["cr_div"][q]
-            parts = _split(list(range(t["cr_ptr"][q], t["cr_ptr"][q + 1]))) or [[]]
+            # (a tail block's own pivots follow the terms in front of it in
+            # batches of their own, cell_sched.tail_size)
+            parts = _split(list(range(t["cr_ptr"][q], t["cr_hd"][q]))) or [[]]
+            parts += _split(list(range(t["cr_hd"][q], t["cr_ptr"][q + 1])))
             for n_, part in enumerate(parts):
                 rd = []
                 for x in part:
@@ -106,8 +111,10 @@ def solve_events(m):
     nv = m["nvar"]
     crow, diag, icol = m["lu_crow"], m["lu_diag"], m["lu_icol"]
 
-    def row(i, lo, hi, extras):
-        for n_, part in enumerate(_split(list(range(lo, hi))) or [[]]):
+    tail = cell_sched.tail_size(m)
+
+    def row(i, ks, nhd, extras):
+        for n_, part in enumerate((_split(ks[:nhd]) or [[]]) + _split(ks[nhd:])):
             rd = []
             for k in part:
                 rd += [k, ("x", icol[k])]
@@ -116,9 +123,13 @@ def solve_events(m):
 
     for i in range(nv):
         if crow[i] != diag[i]:
-            row(i, crow[i], diag[i], [("x", i)])
+            ks = list(range(crow[i], diag[i]))
+            row(i, ks, sum(1 for k in ks if icol[k] < nv - tail), [("x", i)])
     for i in range(nv - 1, -1, -1):
-        row(i, diag[i] + 1, crow[i + 1], [("x", i), diag[i]])
+        ks = list(range(diag[i] + 1, crow[i + 1]))
+        if tail:
+            ks.reverse()
+        row(i, ks, 0 if tail and i >= nv - tail else len(ks), [("x", i), diag[i]])
     return ev
 
 
