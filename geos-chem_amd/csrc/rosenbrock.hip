@@ -441,9 +441,9 @@ __device__ int dev_decomp_crout(CL lu) {
     const int qe = SEG ? M::lu_diag(k) : q1;
 #pragma unroll 1
     for (; q < qe; ++q) {
-      double acc = gather_fma<U>(M::cr_ptr(q), M::cr_ptr(q + 1), (double)lu[q],
-                                 [&](int t) -> double { return -(double)lu[M::cr_l(t)]; },
-                                 [&](int t) -> double { return lu[M::cr_u(t)]; });
+      double acc = gather_sum<M, U>(M::cr_ptr(q), M::cr_hd(q), M::cr_ptr(q + 1), (double)lu[q],
+                                    [&](int t) -> double { return -(double)lu[M::cr_l(t)]; },
+                                    [&](int t) -> double { return lu[M::cr_u(t)]; });
       const int dv = M::cr_div(q);
       if (dv >= 0) acc = acc / lu[dv];
       lu[q] = acc;
@@ -821,7 +821,9 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
     bool singular = true;
     while (singular) {
       dev_jac<M>(Yc, fix, rct, Ascr, LU, -1.0, 1.0 / (dir * H * kRosGamma1));
-      int ising = dev_decomp<M>(LU);
+      int ising;
+      if constexpr (M::TAIL > 0) ising = dev_decomp_crout<M>(LU);  // the order of the cell programs
+      else ising = dev_decomp<M>(LU);
       st[5] += 1;
       if (ising == 0) {
         singular = false;
@@ -862,7 +864,7 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
     }
     // new solution, error estimate (E = (0,0,0,1): Yerr = K4), scaled norm
     double err = 0.0;
-    for (int i = 0; i < N; ++i) {
+    auto err_sum = [&](int i, double &sum) {
       double y0 = Yc[i];
       double v = y0;
       for (int j = 0; j < 4; ++j)
@@ -874,7 +876,16 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
       double ymax = max_f(fabs(y0), fabs(v));
       double sc = P.vectol ? a.atol[i] + a.rtol[i] * ymax : a.atol[0] + a.rtol[0] * ymax;
       double q = ye / sc;
-      err = fma(q, q, err);
+      sum = fma(q, q, sum);
+    };
+    if constexpr (M::TAIL > 0) {  // as the persistent solvers add it
+      for (int l = 0; l < 64; ++l) {
+        double part = 0.0;
+        for (int i = l; i < N; i += 64) err_sum(i, part);
+        err += part;
+      }
+    } else {
+      for (int i = 0; i < N; ++i) err_sum(i, err);
     }
     err = max_f(sqrt(err / N), 1.0e-10);
     double fac = min_f(P.FacMax, max_f(P.FacMin, P.FacSafe / pow(err, 1.0 / kRosELO)));
