@@ -24,17 +24,38 @@ typedef __attribute__((address_space(3))) double lds_double;
 struct CellLds {
   unsigned base, own, coef;
   int lane;
+  __amdgpu_buffer_rsrc_t words;  // the programs' words
 };
 __device__ __forceinline__ double cell_ld(unsigned off) { return *(const lds_double *)off; }
 __device__ __forceinline__ void cell_st(unsigned off, double v) { *(lds_double *)off = v; }
 
-// Block k of a program's words (four words a lane, 1 KB a block).
-__device__ __forceinline__ uint4 cell_word(const unsigned *w, int lane, int k) {
-  return *(const uint4 *)(w + (k * 64 + lane) * 4);
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+// Block k of the programs' words (four words a lane, 1 KB a block), through a
+// buffer resource: the block's offset is a constant, so no load needs an
+// address register (a base address for every four blocks had pushed the
+// kernel's registers into scratch).
+__device__ __forceinline__ u32x4 cell_word(const CellLds &c, int k) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(c.words, c.lane * 16, k * 1024, 0));
 }
-// True on the lanes of a constant mask (the mask goes straight into exec).
-__device__ __forceinline__ bool lanes_of(unsigned long long m) {
-  return __builtin_amdgcn_inverse_ballot_w64(m);
+// True on the lanes of a constant mask.  (The asm keeps the masks out of
+// registers: hoisted from the attempt loop as constants, they spilled.)
+template <unsigned LO, unsigned HI>
+__device__ __forceinline__ bool lanes_of() {
+  unsigned lo, hi;
+  asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"(LO));
+  asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"(HI));
+  return __builtin_amdgcn_inverse_ballot_w64((uint64_t)hi << 32 | lo);
+}
+// x = fma(-t, s, x) on the lanes of a constant mask, s the same on every lane
+// (the wave runs with all lanes on).  One FMA on the chain x -> s -> x; a
+// select would put two more instructions there.
+template <unsigned LO, unsigned HI>
+__device__ __forceinline__ void fma_on(double &x, double t, double s) {
+  asm volatile(
+      "s_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %4\n\tv_fma_f64 %0, -%1, %2, %0\n\t"
+      "s_mov_b64 exec, -1"
+      : "+v"(x)
+      : "v"(t), "s"(s), "i"(LO), "i"(HI));
 }
 // Lane l's value on every lane.
 __device__ __forceinline__ double bcast(double v, int l) {
@@ -46,9 +67,8 @@ __device__ __forceinline__ double bcast(double v, int l) {
 // x / d from y = 1 / d (correctly rounded): Markstein's two-step quotient
 // (IBM J. Res. Dev. 34(1), 1990), the same double as x / d for finite
 // operands away from underflow, in three dependent FMAs where the division
-// sequence takes eleven instructions.  exact: the division itself.
-__device__ __forceinline__ double cell_div(double x, double d, double y, int exact) {
-  if (exact) return x / d;
+// sequence takes eleven instructions.
+__device__ __forceinline__ double cell_div(double x, double d, double y) {
   const double q = x * y;
   return fma(fma(-d, q, x), y, q);
 }
@@ -81,6 +101,9 @@ template <> struct CellProg<Traits_fullchem> {
                                                double yd) {
     cell_fullchem::cell_solve(c, T, ud, yd);
   }
+  static __device__ __forceinline__ __amdgpu_buffer_rsrc_t words() {
+    return brsrc(cell_fullchem::words, (int)sizeof(cell_fullchem::words));
+  }
   static __device__ int rx(int i) { return cell_fullchem::rx[i]; }
   static __device__ double coef(int i) { return cell_fullchem::coef[i]; }
   static __device__ __forceinline__ void constants(const CellLds &c) {
@@ -93,15 +116,14 @@ template <> struct CellProg<Traits_fullchem> {
 };
 
 // What a lane keeps of its wave's cell between attempts: the rate constants
-// of its reactions, and of species lane + 64 k the concentration, Fcn0 and
-// the tolerances.
+// of its reactions, and of species lane + 64 k the concentration and Fcn0.
 template <class M>
 struct CellState {
   static constexpr int KS = (M::NVAR + 63) / 64;
-  double R[CellProg<M>::ROWS], Y[KS], F0[KS], at[KS], rt[KS];
+  double R[CellProg<M>::ROWS], Y[KS], F0[KS];
 };
 
-// Fixed species, rate constants and tolerances of the cell; Y is the
+// Fixed species and rate constants of the cell; Y is the
 // caller's.
 template <class M>
 __device__ __forceinline__ void cell_load(const IntegrateArgs &a, const CellLds &c, int64_t cell,
@@ -114,12 +136,6 @@ __device__ __forceinline__ void cell_load(const IntegrateArgs &a, const CellLds 
 #pragma unroll
   for (int u = 0; u < P::ROWS; ++u)
     s.R[u] = a.rconst[(int64_t)P::rx(u * 64 + c.lane) * a.rstride + cell];
-#pragma unroll
-  for (int k = 0; k < CellState<M>::KS; ++k) {
-    const int i = c.lane + 64 * k < M::NVAR ? c.lane + 64 * k : M::NVAR - 1;
-    s.at[k] = a.atol[a.prm.vectol ? i : 0];
-    s.rt[k] = a.rtol[a.prm.vectol ? i : 0];
-  }
   wave_sync();
 }
 
@@ -270,13 +286,19 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
   const double H = S.H;
   // Ynew and the error norm: a lane's terms in species order, then the 64
   // lanes' sums in lane order
-  double yn[KS], part = 0.0;
+  double yn[KS], at[KS], rt[KS], part = 0.0;
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    const int i = prm.vectol ? (c.lane + 64 * k < N ? c.lane + 64 * k : N - 1) : 0;
+    at[k] = a.atol[i];
+    rt[k] = a.rtol[i];
+  }
 #pragma unroll
   for (int k = 0; k < KS; ++k) {
     yn[k] = fma(1.0, K3[k], fma(1.0, K2[k], fma(2.0, K0[k], cs.Y[k])));
     const double ye = fma(1.0, K3[k], 0.0);
     const double ymax = max_f(fabs(cs.Y[k]), fabs(yn[k]));
-    const double q = ye / (cs.at[k] + cs.rt[k] * ymax);
+    const double q = ye / (at[k] + rt[k] * ymax);
     if (64 * (k + 1) <= N || c.lane + 64 * k < N) part = fma(q, q, part);
   }
   wave_sync();

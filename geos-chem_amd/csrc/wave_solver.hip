@@ -705,6 +705,7 @@ __global__ __launch_bounds__((64 * QueueLds<M0, M1, M2>::WPB), 1) void k_wave(Pe
     cl.base = cl.coef + 8u * (Lds::NCOEF + wib * Lds::SH);
     cl.own = cl.base + 8u * lane;
     cl.lane = lane;
+    cl.words = CellProg<M0>::words();
     __syncthreads();
     if (wave >= pa.nwaves) return;
   }

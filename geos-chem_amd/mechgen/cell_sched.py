@@ -440,14 +440,14 @@ class Stream:
         while len(self.words) % 4:
             self.words.append([0] * LANES)
         nb = len(self.words) // 4
-        out = ["const uint4 w%d = LDW(%d);" % (b, b) for b in range(min(RING, nb))]
+        out = ["const u32x4 w%d = LDW(%d);" % (b, b) for b in range(min(RING, nb))]
         for c in self.code:
             if c[0] != "@":
                 out.append(c)
                 continue
             b = int(c[1:]) + RING - 1
             if b >= RING and b < nb:
-                out.append("const uint4 w%d = LDW(%d);" % (b, b))
+                out.append("const u32x4 w%d = LDW(%d);" % (b, b))
         flat = []
         for b in range(nb):
             for ln in range(LANES):
@@ -518,8 +518,8 @@ def emit_rounds(st, rounds, kind, L, tag):
 
 
 def emit_code(m, t, o):
-    """(C++ text of the generated header's functions, {array: words}, the
-    phases' rounds)."""
+    """(C++ text of the generated header's functions, the words of all its
+    programs, the phases' rounds)."""
     L, k, s, rows, uq = o["layout"], o["tail"], o["s"], o["rows"], o["uq"]
     n, nv = m["nvar"], m["nvar"]
     one = L["ONE"]
@@ -527,15 +527,15 @@ def emit_code(m, t, o):
     at = [None] * (len(rows) * LANES)
     for r, p in enumerate(o["slot"]):
         at[p] = r
-    out, arrays, sched = [], {}, {}
+    out, all_words, sched = [], [], {}
 
-    def func(name, args, st, head=()):
+    def func(name, args, st):
         code, words = st.finish()
-        arrays["cw_%s" % name] = words
         out.append("__device__ __forceinline__ void %s(const CellLds &c%s) {" % (name, args))
-        out.append("#define LDW(k) cell_word(cw_%s, c.lane, k)" % name)
+        out.append("#define LDW(k) cell_word(c, %d + (k))" % (len(all_words) // (4 * LANES)))
         out.extend("  " + x for x in code)
         out.append("#undef LDW\n}")
+        all_words.extend(words)
 
     # Fun: products into A, then Vdot into X
     st = Stream("fun")
@@ -601,18 +601,19 @@ def emit_code(m, t, o):
         st.line("T[%d] = LD(%s & 0xffffu);" % (j, e))
         if j + 1 < k:
             st.line("T[%d] = LD(%s >> 16);" % (j + 1, e))
-    mask = lambda rs: "0x%xull" % sum(1 << i for i in rs)
+    mask = lambda rs: "0x%xu, 0x%xu" % (sum(1 << i for i in rs if i < 32),
+                                        sum(1 << i - 32 for i in rs if i >= 32))
     st.line("ud = 1.0;")
     for j in range(k):
         below = [i for i in range(j + 1, k) if pat[i][j]]
-        st.line("if (lanes_of(%s)) ud = T[%d];" % (mask([j]), j))
+        st.line("if (c.lane == %d) ud = T[%d];" % (j, j))
         if not below:
             continue
         cols = [x for x in range(j + 1, k) if pat[j][x]]
         st.line("{ const double u = bcast(T[%d], %d);" % (j, j))
         for x in cols:
             st.line("const double s%d = bcast(T[%d], %d);" % (x, x, j))
-        st.line("if (lanes_of(%s)) {" % mask(below))
+        st.line("if (lanes_of<%s>()) {" % mask(below))
         st.line("T[%d] = T[%d] / u;" % (j, j))
         for x in cols:
             st.line("T[%d] = fma(-T[%d], s%d, T[%d]);" % (x, j, x, x))
@@ -629,23 +630,23 @@ def emit_code(m, t, o):
     for j in range(k):
         below = [i for i in range(j + 1, k) if pat[i][j]]
         if below:
-            st.line("{ const double s = bcast(x, %d); if (lanes_of(%s)) x = fma(-T[%d], s, x); }"
-                    % (j, mask(below), j))
-    st.line("const double x0 = x; double q = 0.0;")
-    st.line("#pragma unroll 1")
-    st.line("for (int exact = 0; exact < 2; ++exact) {")
+            st.line("fma_on<%s>(x, T[%d], bcast(x, %d));" % (mask(below), j, j))
+    st.line("const double x0 = x;")
+    above = [[i for i in range(j) if pat[i][j]] for j in range(k)]
+    for j in range(k - 1, -1, -1):
+        if above[j]:
+            st.line("fma_on<%s>(x, T[%d], bcast(cell_div(x, ud, yd), %d));" % (mask(above[j]), j, j))
+    st.line("double q = cell_div(x, ud, yd);")
+    st.line("if (__any(q != q)) {  // infinities and NaN: as the division has them")
     st.line("x = x0;")
     for j in range(k - 1, -1, -1):
-        above = [i for i in range(j) if pat[i][j]]
-        if above:
-            st.line("{ q = cell_div(x, ud, yd, exact); const double s = bcast(q, %d); "
-                    "if (lanes_of(%s)) x = fma(-T[%d], s, x); }" % (j, mask(above), j))
-    st.line("q = cell_div(x, ud, yd, exact);")
-    st.line("if (!__any(q != q)) break;")
+        if above[j]:
+            st.line("fma_on<%s>(x, T[%d], bcast(x / ud, %d));" % (mask(above[j]), j, j))
+    st.line("q = x / ud;")
     st.line("}")
     st.line("if (c.lane < %d) STL(%d, q);" % (k, 8 * (L["X"] + s)))
     st.line("wave_sync();")
     sched["sb"] = o["sb"].schedule()
     emit_rounds(st, sched["sb"], "n", L, "b")
     func("cell_solve", ", const double (&T)[%d], double ud, double yd" % k, st)
-    return "\n".join(out), arrays, sched
+    return "\n".join(out), all_words, sched

@@ -235,9 +235,7 @@ def cell_text(name, m, t, cell):
            "constexpr int X0 = %d, ZERO = %d, ONE = %d, NEG = %d, SINK = %d;"
            % (L["X"], L["ZERO"], L["ONE"], L["NEG"], L["SINK"]),
            arr("int", "rx", rx), arr("double", "coef", cell["coef"], per_line=6, fmt=dfmt)]
-    for k, v in words.items():
-        out.append(arr("unsigned", k, v, align=16))
-    out += [code, "}  // namespace cell_%s" % name, ""]
+    out += [arr("unsigned", "words", words, align=16), code, "}  // namespace cell_%s" % name, ""]
     return "\n".join(out)
 
 
