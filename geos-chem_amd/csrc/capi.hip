@@ -130,7 +130,15 @@ extern "C" int gckpp_mech_sizes(int mech_id, int32_t out[8]) {
 
 // Persistent configuration and its launch size: every resident wave, at
 // most one wave per 64 cells of the workspace, a whole number of workgroups.
-static const int kDefaultPersistVariant = 4, kDefaultPersistWpb = 1;
+static const int kDefaultLaneVariant = 4, kDefaultPersistWpb = 1;
+// A context starts with the cell-per-wave kernel where the mechanism has cell
+// programs (fullchem), whatever the number of cells: its attempt takes 61 us
+// on each of 768 waves (337 k cold cells/s), the lane kernel's 24 ms on each
+// of up to 262,144 lanes (135 k cells/s at 238,464 cells, fewer below).  The
+// other mechanisms start on the lane kernel.
+static int default_variant(int mech) {
+  return mech == MECH_FULLCHEM ? PERSIST_WAVE_VARIANT : kDefaultLaneVariant;
+}
 // Waves a persistent launch needs for ncell cells (before the resident cap):
 // a lane-per-cell wave takes 64 cells at a time, a wave-per-cell wave one.
 static int64_t cells_to_waves(int variant, int64_t ncell) {
@@ -240,8 +248,8 @@ extern "C" int gckpp_init(int mech_id, int64_t max_cells, gckpp_ctx **out) {
   for (int k = 0; k < 5; ++k) INIT_OK(hipEventCreate(&c->ev[k]));
   INIT_OK(hipMalloc(&c->counter, sizeof(unsigned int)));
   c->solver = GCKPP_SOLVER_PLAIN;
-  if (set_pconfig(c, kDefaultPersistVariant, kDefaultPersistWpb) != 0) {
-    c->pvariant = kDefaultPersistVariant;
+  if (set_pconfig(c, default_variant(mech_id), kDefaultPersistWpb) != 0) {
+    c->pvariant = kDefaultLaneVariant;
     c->pwpb = 1;
     c->pwaves = c->wstride / 64 < 1024 ? c->wstride / 64 : 1024;
   }
@@ -1302,7 +1310,7 @@ extern "C" int gckpp_autotune_dev(gckpp_ctx *c, int64_t ncell, double tin, doubl
     }
   }
   c->solver = keep_solver;
-  if (set_pconfig(c, best_v, best_g) != 0) set_pconfig(c, kDefaultPersistVariant, 1);
+  if (set_pconfig(c, best_v, best_g) != 0) set_pconfig(c, kDefaultLaneVariant, 1);
   return rc;
 }
 
@@ -1315,7 +1323,9 @@ extern "C" int gckpp_autotune_dev(gckpp_ctx *c, int64_t ncell, double tin, doubl
 struct gckpp_batch {
   gckpp_ctx *ctx[3];      // fullchem, Hg, carbon (null: absent)
   int variant, wpb;
+  bool chosen;            // by gckpp_batch_set_config; else batch_enqueue's rule
   int64_t nwaves, slot_fields;
+  int64_t wave_waves;     // resident waves of the cell-per-wave kernel
   double *work;           // [cap_waves][slot_fields][64]
   int64_t cap_waves;
   int64_t max_waves;      // gckpp_batch_set_waves (0: every resident wave)
@@ -1358,7 +1368,8 @@ extern "C" int gckpp_batch_init(gckpp_ctx *fullchem, gckpp_ctx *hg, gckpp_ctx *c
   auto *b = new gckpp_batch();
   for (int q = 0; q < 3; ++q) b->ctx[q] = cs[q];
   b->slot_fields = persist_slot_fields(PQ_MIXED);
-  if (batch_config(b, kDefaultPersistVariant, 1, 0) != 0) {
+  b->wave_waves = persist_resident_waves(PQ_MIXED, PERSIST_WAVE_VARIANT, 1);
+  if (b->wave_waves <= 0 || batch_config(b, kDefaultLaneVariant, 1, 0) != 0) {
     delete b;
     return fail("gckpp_batch_init: cannot size the persistent launch");
   }
@@ -1418,18 +1429,30 @@ static int batch_enqueue(gckpp_batch *b, const gckpp_part parts[3], double dt, h
     pa.qend[q] = end;
   }
   if (end == 0) return 0;
+  // Without a configuration of the caller's: the cell-per-wave kernel when the
+  // batch has fullchem cells, which then are nearly all of its work (20,011
+  // cells, 70/20/10 %: 50 ms where the lane kernel with the hand-off took
+  // 197 ms), else the lane kernel (64 Hg cells a wave).
+  int variant = b->variant, wpb = b->wpb;
+  int64_t nwaves = b->nwaves;
+  if (!b->chosen && pa.qend[0] > 0) {
+    variant = PERSIST_WAVE_VARIANT;
+    wpb = 1;
+    nwaves = b->wave_waves;
+    if (b->max_waves > 0 && nwaves > b->max_waves) nwaves = b->max_waves;
+  }
   pa.work = b->work;
-  pa.slot_fields = launch_slot_fields(PQ_MIXED, b->variant);
+  pa.slot_fields = launch_slot_fields(PQ_MIXED, variant);
   pa.counter = b->counter;
-  const bool hand = b->ho_cap > 0 && b->ho_rec && b->variant != PERSIST_WAVE_VARIANT;
+  const bool hand = b->ho_cap > 0 && b->ho_rec && variant != PERSIST_WAVE_VARIANT;
   if (hand) {
     launch_zero_u32(b->ho_ctr, 4, s);
     pa.ho = Handoff{b->ho_ctr, b->ho_ctr + 1, b->ho_ctr + 3, b->ho_cell, b->ho_rec, b->ho_cap, 0};
   }
-  int64_t nw = cells_to_waves(b->variant, end);
-  nw = (nw + b->wpb - 1) / b->wpb * b->wpb;
-  if (nw > b->nwaves) nw = b->nwaves;
-  if (launch_persist(PQ_MIXED, b->variant, b->wpb, pa, nw, s) != 0)
+  int64_t nw = cells_to_waves(variant, end);
+  nw = (nw + wpb - 1) / wpb * wpb;
+  if (nw > nwaves) nw = nwaves;
+  if (launch_persist(PQ_MIXED, variant, wpb, pa, nw, s) != 0)
     return fail("gckpp_batch: persistent launch failed: %s", hipGetErrorString(hipGetLastError()));
   if (hand) {
     PersistArgs ph = pa;
@@ -1552,6 +1575,7 @@ extern "C" int gckpp_batch_set_config(gckpp_batch *b, int variant, int waves_per
     return fail("gckpp_batch_set_config: bad variant or waves per workgroup");
   if (batch_config(b, variant, waves_per_group, b->cap_waves) != 0)
     return fail("gckpp_batch_set_config: configuration does not fit");
+  b->chosen = true;
   return 0;
 }
 
