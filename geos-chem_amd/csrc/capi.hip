@@ -1612,7 +1612,7 @@ struct gckpp_mlp {
   unsigned short *packed;                  // [MLP_NPACK] bf16
   bool packed_ok;
   int step;
-  float *act, *dO, *dA, *lossp;            // training scratch for max_batch rows
+  float *act, *dO, *dw, *lossp;            // training scratch for max_batch rows
 };
 
 extern "C" int gckpp_mlp_init(int64_t max_batch, const int32_t jslot[12], const int32_t spc[24],
@@ -1637,8 +1637,8 @@ extern "C" int gckpp_mlp_init(int64_t max_batch, const int32_t jslot[12], const 
       hipMalloc(&m->packed, sizeof(unsigned short) * MLP_NPACK) != hipSuccess ||
       hipMalloc(&m->act, na) != hipSuccess ||
       hipMalloc(&m->dO, sizeof(float) * (size_t)max_batch * MLP_O) != hipSuccess ||
-      hipMalloc(&m->dA, sizeof(float) * (size_t)max_batch * MLP_H) != hipSuccess ||
-      hipMalloc(&m->lossp, sizeof(float) * (size_t)((max_batch + 255) / 256)) != hipSuccess ||
+      hipMalloc(&m->dw, sizeof(float) * (size_t)mlp_dw_floats(max_batch)) != hipSuccess ||
+      hipMalloc(&m->lossp, sizeof(float) * (size_t)mlp_loss_parts(max_batch)) != hipSuccess ||
       hipMemset(m->params, 0, np) != hipSuccess || hipMemset(m->adam_m, 0, np) != hipSuccess ||
       hipMemset(m->adam_v, 0, np) != hipSuccess) {
     gckpp_mlp_finalize(m);  // releases what was allocated (the rest is null)
@@ -1724,8 +1724,8 @@ static int mlp_grad_impl(gckpp_mlp *m, int64_t nb, const float *X, const float *
                          const int32_t *ycls, float wh, float wc, float *loss, hipStream_t s) {
   if (!m || !X || !yh || !ycls) return fail("gckpp_mlp_grad: null argument");
   if (nb <= 0 || nb > m->max_batch) return fail("gckpp_mlp_grad: nb must be in [1, max_batch]");
-  mlp_grad_f32(m->params, nb, X, yh, ycls, wh, wc, m->act, m->dO, m->dA, m->grad, m->lossp, s);
-  if (loss) mlp_sum(m->lossp, (nb + 255) / 256, loss, s);
+  mlp_grad_f32(m->params, nb, X, yh, ycls, wh, wc, m->act, m->dO, m->dw, m->grad, m->lossp, s);
+  if (loss) mlp_sum(m->lossp, mlp_loss_parts(nb), loss, s);
   HIP_OK(hipGetLastError());
   return 0;
 }
@@ -1758,7 +1758,7 @@ extern "C" int gckpp_mlp_finalize(gckpp_mlp *m) {
   if (!m) return 0;
   bool ok = true;
   for (void *p : {(void *)m->params, (void *)m->grad, (void *)m->adam_m, (void *)m->adam_v,
-                  (void *)m->packed, (void *)m->act, (void *)m->dO, (void *)m->dA,
+                  (void *)m->packed, (void *)m->act, (void *)m->dO, (void *)m->dw,
                   (void *)m->lossp})
     if (p) ok = hipFree(p) == hipSuccess && ok;
   delete m;

@@ -47,8 +47,10 @@ void mlp_predict(const MlpDesc &d, int64_t n, const double *met, const double *p
                  int32_t *cls, hipStream_t s);
 void mlp_forward_f32(const float *P, int64_t nb, const float *X, float *act, hipStream_t s);
 void mlp_grad_f32(const float *P, int64_t nb, const float *X, const float *yh, const int32_t *ycls,
-                  float wh, float wc, float *act, float *dO, float *dA, float *G, float *lossp,
+                  float wh, float wc, float *act, float *dO, float *dw, float *G, float *lossp,
                   hipStream_t s);
+int64_t mlp_loss_parts(int64_t nb);  // floats of lossp
+int64_t mlp_dw_floats(int64_t nb);   // floats of dw
 // order[0..n) = cells sorted by class, class 3 first, stable; scratch: 4*ceil(n/256) ints
 void order_by_class(int64_t n, const int32_t *cls, int32_t *order, int32_t *scratch, hipStream_t s);
 // order[0..n) = cells sorted by predicted h0, smallest first (32 bins of
