@@ -69,6 +69,7 @@ struct gckpp_ctx {
   float *hlog;         // persistent solver: step-history log (device), or null
   int hlog_n;
   int pvariant;        // persistent kernel variant (loads in flight x register budget)
+  bool pchosen;        // by the caller (gckpp_set_persistent_config, the autotuner)
   int pwpb;            // waves per workgroup of the persistent launch
   int64_t pwaves;      // waves of one persistent launch (multiple of pwpb)
   int64_t pwaves_max;  // caller's cap on pwaves (0: every resident wave)
@@ -407,10 +408,14 @@ static void fill_persist_queue(const gckpp_ctx *c, IntegrateArgs &a, int64_t nce
 // configured variant on the rest of the order; work later enqueued on s
 // waits for both.  With a hand-off set (lane variants), the lane kernel's
 // last unfinished cells move at a step boundary to a cell-per-wave launch
-// that follows it on s.
+// that follows it on s.  Neither for the unrolled lane kernel (Hg) unless the
+// caller chose its configuration: a cell-per-wave launch has one cell a wave
+// where this one has 64, and the hand-off's list of 98,304 cells took
+// 27 ms of a 50 ms grid step.
 static int launch_persist_queue(gckpp_ctx *c, PersistArgs &pa, int64_t ncell, hipStream_t s,
                                 const char *who) {
-  const bool can_split = c->split > 0 && c->wwork && pa.q[0].order && ncell > c->split &&
+  const bool whole = unrolled_kernel(c->mech) && !c->pchosen;
+  const bool can_split = !whole && c->split > 0 && c->wwork && pa.q[0].order && ncell > c->split &&
                          c->mech != MECH_CARBON && c->pvariant != PERSIST_WAVE_VARIANT;
   const int64_t k = can_split ? c->split : 0;
   if (k > 0) {
@@ -428,7 +433,7 @@ static int launch_persist_queue(gckpp_ctx *c, PersistArgs &pa, int64_t ncell, hi
     pa.q[0].order += k;
     pa.qend[0] = pa.qend[1] = pa.qend[2] = ncell - k;
   }
-  const bool hand = c->ho_cap > 0 && c->ho_rec && c->mech != MECH_CARBON &&
+  const bool hand = !whole && c->ho_cap > 0 && c->ho_rec && c->mech != MECH_CARBON &&
                     c->pvariant != PERSIST_WAVE_VARIANT && ncell - k > 0;
   c->ho_timed = false;  // the statistics describe this solve from here on
   if (hand) {
@@ -1228,6 +1233,7 @@ extern "C" int gckpp_set_persistent_config(gckpp_ctx *c, int variant, int waves_
   if (set_pconfig(c, variant, waves_per_group) != 0)
     return fail("gckpp_set_persistent_config: variant %d with %d waves per workgroup does not fit",
                 variant, waves_per_group);
+  c->pchosen = true;
   return 0;
 }
 
@@ -1314,6 +1320,7 @@ extern "C" int gckpp_autotune_dev(gckpp_ctx *c, int64_t ncell, double tin, doubl
     }
   }
   c->solver = keep_solver;
+  c->pchosen = true;
   if (set_pconfig(c, best_v, best_g) != 0) set_pconfig(c, kDefaultLaneVariant, 1);
   return rc;
 }

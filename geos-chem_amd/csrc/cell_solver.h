@@ -182,11 +182,11 @@ __device__ __forceinline__ void cell_finish(const IntegrateArgs &a, const CellLd
 // of operations); true when the cell is done (S.ierr then holds IERR).
 template <class M>
 __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellLds &c, int64_t cell,
-                                             WaveState &S, CellState<M> &cs) {
+                                             RosState &S, CellState<M> &cs) {
   using P = CellProg<M>;
   constexpr int N = M::NVAR, KS = CellState<M>::KS;
   const RosParams &prm = a.prm;
-  const double Tend = prm.Tend, dir = prm.direction;
+  const double dir = prm.direction;
   // the lane's species of a vector to X and back
   auto put = [&](const double (&v)[KS]) {
     wave_sync();
@@ -202,13 +202,7 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
       v[k] = 64 * (k + 1) <= N || c.lane + 64 * k < N ? LDL(8 * (P::X0 + 64 * k)) : 0.0;
     wave_sync();
   };
-  if (S.newStep) {
-    const bool more = (dir > 0) ? ((S.T - Tend) + prm.roundoff <= 0.0) : ((Tend - S.T) + prm.roundoff <= 0.0);
-    if (!more) return true;
-    if (S.st[2] > prm.max_steps) { S.ierr = -6; return true; }
-    if ((S.T + 0.1 * S.H) == S.T || S.H <= prm.roundoff) { S.ierr = -7; return true; }
-    S.H = min_f(S.H, fabs(Tend - S.T));
-  }
+  if (S.newStep && state_done(prm, S)) return true;
   double K0[KS], K1[KS], K2[KS], K3[KS], T[P::TAIL], ud = 1.0, yd = 1.0, dH = 0.0;
 #pragma unroll
   for (int k = 0; k < KS; ++k) K0[k] = K1[k] = K2[k] = K3[k] = 0.0;
@@ -314,33 +308,13 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
     for (int u = 0; u < 16; ++u) err += q[u];
   }
   err = max_f(sqrt(err / N), 1.0e-10);
-  const double fac = min_f(prm.FacMax, max_f(prm.FacMin, prm.FacSafe / pow(err, 1.0 / kRosELO)));
-  S.Hnew = H * fac;
   if (a.hlog && S.st[2] < a.hlog_n && c.lane == 0) {
     a.hlog[(int64_t)(2 * S.st[2]) * a.ncell + cell] = (float)H;
     a.hlog[(int64_t)(2 * S.st[2] + 1) * a.ncell + cell] = (float)err;
   }
-  S.st[2] += 1;
-  if (err <= 1.0 || H <= prm.Hmin) {
-    S.st[3] += 1;
+  if (state_step(prm, err, S)) {
 #pragma unroll
     for (int k = 0; k < KS; ++k) cs.Y[k] = prm.clip_negative ? max_f(yn[k], 0.0) : yn[k];
-    S.T = S.T + dir * H;
-    S.Hnew = max_f(prm.Hmin, min_f(S.Hnew, prm.Hmax));
-    if (S.rejLast) S.Hnew = min_f(S.Hnew, H);
-    S.Hexit = H;
-    S.Texit = S.T;
-    S.HnewAcc = S.Hnew;
-    S.rejLast = S.rejMore = false;
-    S.H = S.Hnew;
-    S.newStep = true;
-  } else {
-    if (S.rejMore) S.Hnew = H * prm.FacRej;
-    S.rejMore = S.rejLast;
-    S.rejLast = true;
-    S.H = S.Hnew;
-    if (S.st[3] >= 1) S.st[4] += 1;
-    S.newStep = false;
   }
   return false;
 }

@@ -148,6 +148,10 @@ struct WaveKernel {
   size_t lds(int wpb) const { return sizeof(double) * (size_t)(lds_group + wpb * lds_wave); }
 };
 WaveKernel wave_kernel(int qset);
+// The unrolled lane-per-cell kernel of a single-mechanism queue set that has
+// one (Hg; null: none), and the bytes of LDS a wave of it needs.
+const void *unrolled_kernel(int qset);
+constexpr size_t kUnrolledLds = 160 * 64 * sizeof(double);
 int64_t wave_scratch_fields(int qset);  // its global scratch per wave, fields of 64 doubles
 int64_t persist_slot_fields(int qset);                   // doubles per lane slot
 int64_t persist_resident_waves(int qset, int variant, int wpb);  // 0 on error

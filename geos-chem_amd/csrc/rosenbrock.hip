@@ -1496,7 +1496,6 @@ template <int U, int W, bool SEG, int CS = 0>
 static const void *persist_kernel(int qset) {
   switch (qset) {
     case PQ_FULLCHEM: return (const void *)k_persist<U, W, SEG, CS, Traits_fullchem, void, void>;
-    case PQ_HG: return (const void *)k_persist<U, W, SEG, CS, Traits_Hg, void, void>;
     case PQ_CARBON: return (const void *)k_persist<U, W, SEG, CS, Traits_carbon, void, void>;
     case PQ_MIXED:
       return (const void *)k_persist<U, W, SEG, CS, Traits_fullchem, Traits_Hg, Traits_carbon>;
@@ -1507,6 +1506,12 @@ static const void *persist_kernel(int qset) {
 // (register budget), flat segment execution of the independent sums,
 // operand-cache slots per lane
 const void *persist_kernel_variant(int qset, int variant) {
+  // a mechanism with an unrolled kernel (Hg) runs it for every lane variant:
+  // the table walk's loads in flight, segments and operand caches have nothing
+  // to do there, and the slowest unrolled launch beats them all
+  if (variant != PERSIST_WAVE_VARIANT && variant >= 0 && variant < PERSIST_VARIANTS &&
+      unrolled_kernel(qset))
+    return unrolled_kernel(qset);
   switch (variant) {
     case 0: return persist_kernel<1, 1, false>(qset);
     case 1: return persist_kernel<8, 1, false>(qset);
@@ -1547,6 +1552,12 @@ int64_t persist_slot_fields(int qset) {
   }
   return 0;
 }
+// Dynamic LDS of a lane variant's workgroup of wpb waves.
+static size_t lane_lds(int qset, int variant, int wpb) {
+  if (unrolled_kernel(qset)) return kUnrolledLds;  // launched a wave a workgroup
+  const int cs = persist_variant_cache(variant);
+  return cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
+}
 // Resident waves of one launch with wpb waves per workgroup: CUs x the
 // occupancy the variant's register use allows (0 on error).
 int64_t persist_resident_waves(int qset, int variant, int wpb) {
@@ -1555,14 +1566,16 @@ int64_t persist_resident_waves(int qset, int variant, int wpb) {
   if (!k || hipGetDevice(&dev) != hipSuccess) return 0;
   if (variant == PERSIST_WAVE_VARIANT && wpb != 1) return 0;  // its workgroup is one wave
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  const int cs = persist_variant_cache(variant);
-  size_t lds = cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
+  size_t lds = lane_lds(qset, variant, wpb);
+  const int ask = wpb;  // the caller's unit of waves
   if (variant == PERSIST_WAVE_VARIANT) {
     wpb = wave_kernel(qset).max_wpb;
     lds = wave_kernel(qset).lds(wpb);
+  } else if (unrolled_kernel(qset)) {
+    wpb = 1;
   }
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 64 * wpb, lds) != hipSuccess) return 0;
-  return (int64_t)ncu * (per > 0 ? per : 1) * wpb;
+  return (int64_t)ncu * (per > 0 ? per : 1) * wpb / ask * ask;
 }
 // Cell-per-wave launches up to this many waves take a workgroup for each wave:
 // two one-wave workgroups fit a CU, so 256 CUs still hold them all at once,
@@ -1581,8 +1594,7 @@ int launch_persist(int qset, int variant, int wpb, const PersistArgs &args0, int
   if (variant == PERSIST_WAVE_VARIANT && wpb != 1) return -1;
   if (pa.counter) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, pa.counter);
   void *args[] = {(void *)&pa};
-  const int cs = persist_variant_cache(variant);
-  size_t lds = cs ? (size_t)64 * wpb * (cs + 1) * sizeof(double) : 0;
+  size_t lds = lane_lds(qset, variant, wpb);
   int64_t blocks = nwaves / wpb;
   if (variant == PERSIST_WAVE_VARIANT) {
     // few waves: a workgroup (and so a CU's LDS) for each
@@ -1590,6 +1602,9 @@ int launch_persist(int qset, int variant, int wpb, const PersistArgs &args0, int
     wpb = nwaves > kWaveSpread ? w.max_wpb : 1;
     lds = w.lds(wpb);
     blocks = (nwaves + wpb - 1) / wpb;
+  } else if (unrolled_kernel(qset)) {
+    wpb = 1;
+    blocks = nwaves;
   }
   return hipLaunchKernel(k, dim3((unsigned)blocks), dim3(64 * wpb), args, lds, s) ==
                  hipSuccess

@@ -22,6 +22,7 @@
 
 #include "gckpp_internal.h"
 #include "mech_traits.h"
+#include "ros_state.h"
 
 namespace gckpp {
 namespace {
@@ -187,13 +188,6 @@ __device__ __forceinline__ void run_prog(char *shb, const WProg &p, int lane,
   wave_sync();
 }
 
-// Per-cell integrator state, the same on every lane.
-struct WaveState {
-  double T, H, Hnew, Hexit, Texit, HnewAcc;
-  int st[8];
-  int ierr, tries;
-  bool rejLast, rejMore, newStep;
-};
 
 // The cell a wave works on: LDS block sh (layout WV_* of the mechanism) and
 // the wave's global scratch g (WV_G_*): rate constants [NREACT], reaction
@@ -344,25 +338,6 @@ __device__ __forceinline__ void wave_zero_slots(const WaveCell<M> &c) {
   }
 }
 
-// The integrator state at the start of a cell's integration.
-__device__ __forceinline__ void state_begin(const IntegrateArgs &a, int64_t cell, bool cold,
-                                            WaveState &S) {
-  const RosParams &P = a.prm;
-  const double hs = (a.hstart && !cold) ? a.hstart[cell] : 0.0;
-  double Hstart = P.Hstart_default;
-  if (hs > 0.0) Hstart = min_f(fabs(hs), fabs(P.Tend - P.Tstart));
-  S.T = P.Tstart;
-  double H = min_f(max_f(fabs(P.Hmin), fabs(Hstart)), fabs(P.Hmax));
-  if (fabs(H) <= 10.0 * P.roundoff) H = P.DeltaMin;
-  S.H = P.direction * H;
-  S.Hnew = S.H;
-  S.Hexit = S.Texit = S.HnewAcc = 0.0;
-  for (int k = 0; k < 8; ++k) S.st[k] = 0;
-  S.ierr = 1;
-  S.rejLast = S.rejMore = false;
-  S.newStep = true;
-}
-
 template <class M>
 __device__ void wave_begin(const IntegrateArgs &a, const WaveCell<M> &c, int64_t cell) {
   double *sh = c.sh;
@@ -380,7 +355,7 @@ __device__ void wave_begin(const IntegrateArgs &a, const WaveCell<M> &c, int64_t
 // when the cell is done (S.ierr then holds IERR).
 template <class M>
 __device__ bool wave_attempt(const IntegrateArgs &a, const WaveCell<M> &c, int64_t cell,
-                             WaveState &S) {
+                             RosState &S) {
   constexpr int N = M::NVAR;
   constexpr int KS = (N + 63) / 64;  // species per lane: i = lane + 64 k
   double *sh = c.sh;
@@ -559,7 +534,7 @@ __device__ bool wave_attempt(const IntegrateArgs &a, const WaveCell<M> &c, int64
 
 // The carbon mechanism's forward-Euler integration (lane_euler's algorithm).
 template <class M>
-__device__ void wave_euler(const IntegrateArgs &a, const WaveCell<M> &c, WaveState &S) {
+__device__ void wave_euler(const IntegrateArgs &a, const WaveCell<M> &c, RosState &S) {
   double *sh = c.sh;
   wave_fun<M>(c, M::WV_Y0);
   const double dt = a.prm.Tend - a.prm.Tstart;
@@ -585,7 +560,7 @@ __device__ void wave_euler(const IntegrateArgs &a, const WaveCell<M> &c, WaveSta
 // idx of the hand-off list; see Handoff).  Y of the variable species is in
 // the list too; the fixed species and the rate constants come from conc and
 // rconst as at the start of a cell.
-__device__ __forceinline__ void state_resume(const Handoff &ho, int64_t idx, WaveState &S) {
+__device__ __forceinline__ void state_resume(const Handoff &ho, int64_t idx, RosState &S) {
   const double *r = ho.rec + idx;
   const int64_t cap = ho.cap;
   S.T = r[0];
@@ -631,7 +606,7 @@ __device__ void wave_finish(const IntegrateArgs &a, const WaveCell<M> &c, int64_
 }
 
 __device__ __forceinline__ void state_finish(const IntegrateArgs &a, int k, int64_t cell,
-                                             const WaveState &S) {
+                                             const RosState &S) {
   int stk = 0;  // S.st[k] without a lane-indexed (scratch) array access
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -719,7 +694,7 @@ __global__ __launch_bounds__((64 * QueueLds<M0, M1, M2>::WPB), 1) void k_wave(Pe
   int64_t cell = -1;
   int q = 0;
   int64_t next_static = wave;
-  WaveState S;
+  RosState S;
   auto begin = [&](bool cold) {
     on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
       using M = std::remove_pointer_t<decltype(tag)>;

@@ -31,6 +31,7 @@ from pathlib import Path
 sys.path.insert(0, str(Path(__file__).resolve().parent))
 import cell_sched  # noqa: E402
 import lane_cache  # noqa: E402
+import unroll  # noqa: E402
 import wave_sched  # noqa: E402
 
 HERE = Path(__file__).resolve().parent
@@ -301,6 +302,13 @@ def emit(name):
     cell = cell_sched.build(m, t)
     if cell:
         (gen / ("cell_%s.h" % name)).write_text(cell_text(name, m, t, cell))
+    if unroll.fits(m):
+        (gen / ("unroll_%s.h" % name)).write_text("\n".join([
+            "/* Generated by geos-chem_amd/mechgen/emit_tables.py from mech/%s.json"
+            " -- do not edit. */" % name, "#pragma once", "", "namespace unroll_%s {" % name,
+            "constexpr int LDS_FIELDS = %d, NLU_LDS = %d, NRATE_LDS = %d;"
+            % ((unroll.LDS_FIELDS,) + unroll.layout(m)),
+            unroll.code(m, t), "}  // namespace unroll_%s" % name, ""]))
     print("%s: NFV=%d NPART=%d NJV=%d NLE=%d NLP=%d" % (name, len(t["fv_r"]), len(t["pt_r"]),
                                                        len(t["jv_b"]), len(t["le_kk"]), len(t["lp_dst"])))
 
