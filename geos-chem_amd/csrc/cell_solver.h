@@ -11,7 +11,7 @@
 // chain, the last 34 rows -- a chain of pivots -- in registers, and the
 // reaction products in LDS over the tail block's slots (gathered from L2 they
 // cost 64 cache lines a step).  Measured on the 24x23x72 grid, cold step of
-// 39,744 cells: 537 ms with the block programs of wave_sched.py, 118 ms here;
+// 39,744 cells: 537 ms with the block programs of wave_sched.py, 112 ms here;
 // 63 us an attempt and wave where it was 280 us; one cell's Integrate 9.2 ms
 // and 2.8 ms.
 //

@@ -98,6 +98,11 @@ def partial_batches(m):
     return {x: i // AB_ROWS for i, x in enumerate(uq)}, uq
 
 
+# Phase.schedule's candidates.
+POLICIES = ((32, 1, 0.0, 0, 24), (12, 3, 0.0, 48, 24), (24, 1, 0.5, 0, 40), (16, 2, 0.5, 0, 0),
+            (8, 1, 0.125, 0, 24), (10, 1, 0.125, 0, 24), (3, 1, 0.0, 0, 24))
+
+
 class Job:
     """One chunk of a sum: lds[dest] = lds[init] + its terms (/ lds[div]);
     `need`: elements a step or the division reads that another job makes."""
@@ -170,17 +175,19 @@ class Phase:
         terms, those with the longest path to the phase's end first, and runs
         the same number of steps of each (fewer where a job has no more)."""
         # (most steps in a round, fewest worth a piece, how far the longest
-        # path sets a round's steps, divisions that make a round)
+        # path sets a round's steps, divisions that make a round, jobs apart
+        # from the last round that make a round): each the best for one of
+        # fullchem's phases (modelled clocks of an attempt's LU 24.7k -> 16.3k,
+        # Vdot 3.6k -> 2.6k, Jacobian 10.6k -> 9.1k by the rounds apart)
         best = None
-        for policy in ((4, 1, 0.0, 0), (12, 1, 0.5, 0), (12, 3, 0.0, 48), (32, 1, 0.0, 0),
-                       (32, 1, 0.5, 0), (32, 1, 1.0, 0)):
+        for policy in POLICIES:
             r = self._try(*policy)
             if best is None or r[0] < best[0]:
                 best = r
         self.clocks = best[0]
         return best[1]
 
-    def _try(self, cap, minp, share, divs):
+    def _try(self, cap, minp, share, divs, apart):
         jobs, maker = self.jobs, self.maker
         nj = len(jobs)
         # producers of every job's steps and division
@@ -231,6 +238,19 @@ class Phase:
                 cand.append((k, n, fin))
                 if len(cand) >= 6 * LANES:
                     break
+            if apart and rounds:
+                # jobs that need nothing of the last round do not wait for it:
+                # they make the round when they nearly fill it
+                r1 = len(rounds) - 1
+
+                def free(c):
+                    j = jobs[c[0]]
+                    return last[c[0]] < r1 and \
+                        all(done[q] < r1 for x in range(j.pos, j.pos + c[1]) for q in prod[c[0]][x]) and \
+                        not (c[2] and divp[c[0]] >= 0 and done[divp[c[0]]] >= r1)
+                sub = [c for c in cand if free(c)]
+                if len(sub) >= apart:
+                    cand = sub
             crit = jobs[cand[0][0]].height > 1.2 * T_STEP * left / LANES
             keep = [c for c in cand if c[2] or c[1] >= minp] or cand[:1]
             # divs: divisions have rounds of their own, begun when that many
