@@ -3,8 +3,13 @@
 #include "species_Hg.h"
 
 namespace gckpp {
-// Update_RCONST of mechanism Hg: rc[r*rs] for r = 0..93
-GCKPP_HD void rates_Hg(const rl::RateEnv &E, double *rc, int64_t rs) {
+// Update_RCONST of mechanism Hg: rc[r*rs] for r = 0..93, in parts
+constexpr int RATE_PARTS_Hg = 1;
+template <int P>
+__device__ void rates_Hg(const rl::RateEnv &E, double *__restrict__ rc, int64_t rs);
+template <>
+__device__ __forceinline__ void rates_Hg<0>(const rl::RateEnv &E, double *__restrict__ rc,
+    int64_t rs) {
   rc[0 * rs] = (rl::GCARR_ab(E, 1.46e-32,1.86e0)*E.NUMDEN);
   rc[1 * rs] = (rl::GCARR_abc(E, 1.6e-9,1.86e0,-7801.0e0)*E.NUMDEN);
   rc[2 * rs] = (3.9e-11);

@@ -56,6 +56,57 @@ def translate(expr, mech):
     return "".join(out)
 
 
+# Parts of a rate program, a wave each: short enough for the instruction cache,
+# a grid's waves many times what the GPU holds (4 parts, the copies last,
+# 1.61 ms for a call on 238,464 cells; 8 to 20 parts 1.04 to 1.03).
+PARTS = {"fullchem": 8}
+
+
+def weight(stmt):
+    """Rough cost of a statement, in instructions."""
+    if re.search(r"[uU]ptk|Brkd|Hyd|hyp|By", stmt):
+        return 600
+    if "rl::" not in stmt:
+        return 12
+    return 60 if "GCARR_ac(" in stmt or "ARRPLUS_ade(" in stmt else 400
+
+
+def parts(mech, stmts):
+    """[[(reaction, statement)]]: statements with the same arguments side by
+    side (a law's exponentials are evaluated once for all that share them), the
+    heterogeneous laws in parts of their own (divergent, many registers), the
+    copies of constants and inputs spread evenly (memory beside arithmetic)."""
+    n = PARTS.get(mech, 1)
+    idx = list(enumerate(stmts))
+    if n == 1:
+        return [idx]
+
+    def key(x):
+        r, s = x
+        w = weight(s)
+        args = re.findall(r"[-+]?\d[\d.]*e?[-+]?\d*", s.split("(E", 1)[-1])
+        if w == 60:  # a0 exp(c0 / T): by c0
+            return (2, args[-1], s, r)
+        if w == 400:  # by arguments, then law (GC_NIT and GC_ALK share theirs)
+            return (1, ",".join(args), s, r)
+        return (0 if w == 600 else 3, "", "", r)
+
+    laws = sorted((x for x in idx if weight(x[1]) > 12), key=key)
+    copies = [x for x in idx if weight(x[1]) <= 12]
+    total, out, acc = sum(weight(s) for r, s in laws), [[]], 0
+    for x in laws:
+        if acc >= total * len(out) / n:
+            out.append([])
+        out[-1].append(x)
+        acc += weight(x[1])
+    # the copies evenly between every part's laws
+    for p, xs in enumerate(out):
+        cs = copies[len(copies) * p // n:len(copies) * (p + 1) // n]
+        m = [((i + 0.5) / len(l), x) for l in (xs, cs) for i, x in enumerate(l)]
+        out[p] = [x for _, x in sorted(m)]
+    return out
+
+
 def emit(mech):
     m = json.loads((HERE.parent / "mech" / ("%s.json" % mech)).read_text())
     gen = HERE.parent / "csrc" / "gen"
@@ -72,12 +123,19 @@ def emit(mech):
          " -- do not edit. */" % mech, "#pragma once",
          '#include "species_%s.h"' % mech, "",
          "namespace gckpp {",
-         "// Update_RCONST of mechanism %s: rc[r*rs] for r = 0..%d"
-         % (mech, m["nreact"] - 1),
-         "GCKPP_HD void rates_%s(const rl::RateEnv &E, double *rc, int64_t rs) {" % mech]
-    for r, rx in enumerate(m["reactions"]):
-        R.append("  rc[%d * rs] = %s;" % (r, translate(rx["rate"], mech)))
-    R += ["}", "}  // namespace gckpp"]
+         "// Update_RCONST of mechanism %s: rc[r*rs] for r = 0..%d, in parts"
+         % (mech, m["nreact"] - 1)]
+    ps = parts(mech, [translate(rx["rate"], mech) for rx in m["reactions"]])
+    R += ["constexpr int RATE_PARTS_%s = %d;" % (mech, len(ps)),
+          "template <int P>",
+          "__device__ void rates_%s(const rl::RateEnv &E, double *__restrict__ rc, int64_t rs);" % mech]
+    for p, xs in enumerate(ps):
+        R += ["template <>",
+              "__device__ __forceinline__ void rates_%s<%d>(const rl::RateEnv &E, double *__restrict__ rc,"
+              % (mech, p), "    int64_t rs) {"]
+        R += ["  rc[%d * rs] = %s;" % x for x in xs]
+        R += ["}"]
+    R += ["}  // namespace gckpp"]
     (gen / ("rates_%s.h" % mech)).write_text("\n".join(R) + "\n")
     print("%s: %d rate statements" % (mech, m["nreact"]))
 
