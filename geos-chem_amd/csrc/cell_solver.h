@@ -4,16 +4,17 @@
 // stage vectors and the LU's tail block live in the lanes' registers.
 //
 // What bounds it: the LDS round trips of the levels in front of the tail block
-// and the operand reads, two per FMA (about 2,600 LDS reads an attempt), with
+// and the operand reads, two per FMA (about 2,100 LDS reads an attempt), with
 // one wave per SIMD to hide them.  Hence straight-line programs (no flags, no
-// loop control: 14.7k instructions, the operands of six steps in flight), sums
+// loop control: 14.0k instructions, the operands of six steps in flight), sums
 // cut into 32-term chunks so that a 384-term row is not one lane's serial
 // chain, the last 34 rows -- a chain of pivots -- in registers, and the
 // reaction products in LDS over the tail block's slots (gathered from L2 they
-// cost 64 cache lines a step).  Measured on the 24x23x72 grid, cold step of
-// 39,744 cells: 537 ms with the block programs of wave_sched.py, 112 ms here;
-// 63 us an attempt and wave where it was 280 us; one cell's Integrate 9.2 ms
-// and 2.8 ms.
+// cost 64 cache lines a step), and the LU laid out in the order in which the
+// substitutions read it, a step's lanes side by side (112 ms without).
+// Measured on the 24x23x72 grid, cold step of 39,744 cells: 537 ms with the
+// block programs of wave_sched.py, 103 ms here; 55 us an attempt and wave where
+// it was 280 us; one cell's Integrate 9.2 ms and 2.3 ms.
 //
 // Included by wave_solver.hip inside namespace gckpp.
 #pragma once
@@ -35,7 +36,8 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // address register (a base address for every four blocks had pushed the
 // kernel's registers into scratch).
 __device__ __forceinline__ u32x4 cell_word(const CellLds &c, int k) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(c.words, c.lane * 16, k * 1024, 0));
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                       c.words, c.lane * 16 + (k & 3) * 1024, (k >> 2) * 4096, 0));
 }
 // True on the lanes of a constant mask.  (The asm keeps the masks out of
 // registers: hoisted from the attempt loop as constants, they spilled.)

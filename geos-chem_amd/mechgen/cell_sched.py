@@ -37,8 +37,9 @@ consumed in batches of AB rows, and the Jacobian's terms are ordered by batch
 
 A phase's words (one 32-bit word per lane and use, two 16-bit byte offsets
 into the wave's LDS): per round a header (destination, initial value), the
-divisor in a dividing round, then one word per step (a, b).  Four words make a
-block, 64 lanes x 16 bytes.
+divisor in a dividing round, then one word per step (a, b), or half a word (b)
+where the lanes' a lie side by side (`solve_order`).  Four words make a block,
+64 lanes x 16 bytes.
 """
 LANES = 64
 CHUNK = 32
@@ -314,12 +315,34 @@ def build(m, t):
     k = tail_size(m)
     if not k:
         return None
+    return _build(m, t, k, solve_order(_build(m, t, k, [])))
+
+
+def solve_order(o):
+    """LU positions in front of the tail block in the order in which the
+    substitutions' steps read them, a step's lanes side by side: a lane then
+    reads its factor at a fixed offset from its own slot (no address, no bank
+    conflict), and the word of the step names the other operand only."""
+    pos = {p: q for q, p in o["lu"].items() if p < o["layout"]["LUH"]}
+    order, seen = [], set()
+    for rd in o["sf"].schedule() + o["sb"].schedule():
+        for x in range(rd.steps):
+            es = [p.terms[x][0] for p in rd.pieces if x < len(p.terms)]
+            if all(e in pos and e not in seen for e in es):
+                order += [pos[e] for e in es]
+                seen.update(es)
+    return order
+
+
+def _build(m, t, k, order):
+    """`order`: LU positions that lie first, in this order."""
     n, nspec, nz = m["nvar"], m["nspec"], m["lu_nonzero"]
     s = n - k
     crow, diag, icol, irow = m["lu_crow"], m["lu_diag"], m["lu_icol"], m["lu_irow"]
     head = [q for q in range(nz) if not (irow[q] >= s and icol[q] >= s)]
     tail = [q for q in range(nz) if irow[q] >= s and icol[q] >= s]
-    lu = {q: p for p, q in enumerate(head + tail)}
+    first = set(order)
+    lu = {q: p for p, q in enumerate(order + [q for q in head if q not in first] + tail)}
     slot, rows = reaction_rows(m)
     batch, uq = partial_batches(m)
     coefs, cidx = [-0.0], {}
@@ -406,6 +429,8 @@ def build(m, t):
         tt = [(lu[t["cr_l"][x]], lu[t["cr_u"][x]]) for x in xs]
         ph.add(lu[q], lu[q] if q in written else ZERO, tt, div)
         written.add(q)
+    # a step's idle lanes read what lies after its factors, times 0
+    assert written.issuperset(head) and len(head) - len(order) >= LANES
     out["lup"] = ph
     # the tail block: slot of (row, column), ZERO where the pattern has none
     out["tailslot"] = [[ZERO] * k for _ in range(k)]
@@ -441,7 +466,7 @@ class Stream:
     are issued RING blocks ahead."""
 
     def __init__(self, name):
-        self.name, self.words, self.code, self.used = name, [], [], 0
+        self.name, self.words, self.code, self.open = name, [], [], None
 
     def line(self, s):
         self.code.append(s)
@@ -453,6 +478,15 @@ class Stream:
             self.line("@%d" % (i // 4))
         self.words.append(list(lanes))
         return "w%d.%s" % (i // 4, "xyzw"[i % 4])
+
+    def half(self, lanes):
+        """The expression of a 16-bit value per lane, two to a word."""
+        if self.open is None:
+            self.open = (len(self.words), self.word(lanes))
+            return "(%s & 0xffffu)" % self.open[1]
+        (i, e), self.open = self.open, None
+        self.words[i] = [w | x << 16 for w, x in zip(self.words[i], lanes)]
+        return "(%s >> 16)" % e
 
     def finish(self):
         """Code lines with the block loads in place, and the words as uint4
@@ -508,6 +542,15 @@ def emit_rounds(st, rounds, kind, L, tag):
                 st.line("const double d%s = LD(%s);" % (n, st.word(d)))
         elif k == "T":
             w = []
+            fs = [p.terms[x][0] for p in rd.pieces if x < len(p.terms)]
+            if kind == "n" and fs[-1] < L["LUH"] and fs == list(range(fs[0], fs[0] + len(fs))) and \
+                    all(x < len(p.terms) for p in rd.pieces[:len(fs)]):
+                for ln in range(LANES):
+                    t = rd.pieces[ln].terms if ln < len(fs) else []
+                    w.append(8 * (t[x][1] if t else zero))
+                st.line("const double a%s_%d = LDL(%d), b%s_%d = LD%s;"
+                        % (n, x, 8 * fs[0], n, x, st.half(w)))
+                return
             for ln in range(LANES):
                 t = rd.pieces[ln].terms if ln < len(rd.pieces) else []
                 a, b = t[x] if x < len(t) else pad

@@ -57,8 +57,8 @@ def translate(expr, mech):
 
 
 # Parts of a rate program, a wave each: short enough for the instruction cache,
-# a grid's waves many times what the GPU holds (4 parts, the copies last,
-# 1.61 ms for a call on 238,464 cells; 8 to 20 parts 1.04 to 1.03).
+# a grid's waves many times what the GPU holds (a call on 238,464 cells: 8 to 20
+# parts 1.04 to 1.03 ms).
 PARTS = {"fullchem": 8}
 
 
