@@ -1,0 +1,76 @@
+"""Edges of the dispatch between the solvers' kernels, bit by bit.
+
+fullchem solves start on the cell-per-wave kernel, one wave to a workgroup up
+to 512 cells and three above; Hg solves on the unrolled lane kernel, 64 cells
+a wave and two waves a CU.  Every kernel does the same operations in the same
+order, so the tolerance is zero.  The rate program runs in parts of 64 cells:
+a cell's rates do not depend on the call's size.
+"""
+import numpy as np
+import pytest
+
+from gckpp_amd import options
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_dev():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch
+
+
+def _t(torch, a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dtype=torch.float64)
+
+
+@pytest.fixture(scope="module")
+def inputs(torch_dev, fullchem, hg):
+    """(workload, rates of all its cells) per mechanism."""
+    from gckpp_amd import hip, synth
+    from pathlib import Path
+    w = synth.box_cells(fullchem, 1024, 7)
+    ctx = hip.Context(fullchem, 1024)
+    rct = ctx.rates(*(_t(torch_dev, x) for x in (w.met, w.photol, w.het, w.conc))).cpu().numpy()
+    ctx.close()
+    g = dict(np.load(Path(__file__).resolve().parent / "golden" / "Hg_box.npz"))
+    return {"fullchem": (w, w.conc, rct), "Hg": (None, g["conc"], g["rconst"])}
+
+
+@pytest.mark.parametrize("name,variant,n", [("fullchem", 4, n) for n in (1, 2, 511, 512, 513, 515, 769)] +
+                         [("Hg", 7, n) for n in (1, 63, 64, 65, 1000)])
+def test_default_kernel_equals_the_other(name, variant, n, inputs, mech_of, torch_dev):
+    print("case: %s, %d cells, default kernel against variant %d" % (name, n, variant), flush=True)
+    from gckpp_amd import hip
+    m = mech_of(name)
+    _, conc, rct = inputs[name]
+    cells = (np.arange(n) * 37) % conc.shape[1]
+    scale = 1.0 + 1.0e-3 * (np.arange(n) // conc.shape[1])
+    ic, rc = options.fullchem_icntrl()
+    out = []
+    for v in (None, variant):
+        ctx = hip.Context(m, max(n, 64))
+        ctx.set_solver(hip.SOLVER_PERSISTENT)
+        if v is not None:
+            ctx.set_persistent_config(v, 1)
+        c = _t(torch_dev, conc[:, cells] * scale)
+        ist, rst, ierr = ctx.integrate(c, _t(torch_dev, rct[:, cells]), _t(torch_dev, np.zeros(n)), 0.0, 1200.0, ic, rc)
+        out.append([x.cpu().numpy() for x in (c, ist, rst, ierr)])
+        ctx.close()
+    assert (out[0][3] == 1).mean() > 0.9
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 769])
+def test_rates_do_not_depend_on_the_number_of_cells(n, inputs, fullchem, torch_dev):
+    from gckpp_amd import hip
+    w, _, rct = inputs["fullchem"]
+    het = w.het if w.het.ndim == 1 or w.het.shape[1] == 1 else w.het[:, :n]
+    ctx = hip.Context(fullchem, 1024)
+    r = ctx.rates(_t(torch_dev, w.met[:, :n]), _t(torch_dev, w.photol[:, :n]), _t(torch_dev, het),
+                  _t(torch_dev, w.conc[:, :n])).cpu().numpy()
+    ctx.close()
+    assert np.array_equal(r, rct[:, :n])
