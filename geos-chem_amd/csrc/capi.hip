@@ -133,8 +133,8 @@ extern "C" int gckpp_mech_sizes(int mech_id, int32_t out[8]) {
 // most one wave per 64 cells of the workspace, a whole number of workgroups.
 static const int kDefaultLaneVariant = 4, kDefaultPersistWpb = 1;
 // A context starts with the cell-per-wave kernel where the mechanism has cell
-// programs (fullchem), whatever the number of cells: its attempt takes 61 us
-// on each of 768 waves (337 k cold cells/s), the lane kernel's 24 ms on each
+// programs (fullchem), whatever the number of cells: its attempt takes 55 us
+// on each of 768 waves (387 k cold cells/s), the lane kernel's 24 ms on each
 // of up to 262,144 lanes (135 k cells/s at 238,464 cells, fewer below).  The
 // other mechanisms start on the lane kernel.
 static int default_variant(int mech) {

@@ -6,14 +6,14 @@
 // What bounds it: the LDS round trips of the levels in front of the tail block
 // and the operand reads, two per FMA (about 2,100 LDS reads an attempt), with
 // one wave per SIMD to hide them.  Hence straight-line programs (no flags, no
-// loop control: 14.0k instructions, the operands of six steps in flight), sums
+// loop control: 14.0k instructions, the operands of seven steps in flight), sums
 // cut into 32-term chunks so that a 384-term row is not one lane's serial
 // chain, the last 34 rows -- a chain of pivots -- in registers, and the
 // reaction products in LDS over the tail block's slots (gathered from L2 they
 // cost 64 cache lines a step), and the LU laid out in the order in which the
 // substitutions read it, a step's lanes side by side (112 ms without).
 // Measured on the 24x23x72 grid, cold step of 39,744 cells: 537 ms with the
-// block programs of wave_sched.py, 103 ms here; 55 us an attempt and wave where
+// block programs of wave_sched.py, 101 ms here; 55 us an attempt and wave where
 // it was 280 us; one cell's Integrate 9.2 ms and 2.3 ms.
 //
 // Included by wave_solver.hip inside namespace gckpp.

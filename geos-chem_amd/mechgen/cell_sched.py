@@ -46,8 +46,8 @@ CHUNK = 32
 KCELLS = 3              # cells (waves) per CU, the most the LU block leaves room for
 LDS_BYTES = 163840      # per CU
 AB_ROWS = 8             # rows of 64 partials per batch
-RING = 8                # word blocks in flight (L2 latency over about 80 clocks a block)
-DEPTH = 6               # steps whose operands are in flight (lgkmcnt counts 15 reads)
+RING = 12               # word blocks in flight (8: 1 % slower)
+DEPTH = 7               # steps whose operands are in flight (lgkmcnt counts 15 reads)
 
 
 def _pattern(m):
