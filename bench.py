@@ -548,7 +548,8 @@ def warm_legs(args, mech, w, ctx, model, P, ic, rc):
     out["attempts_saved_frac"] = round(1.0 - out["learned"]["mean_attempts"] /
                                        out["plain_kpphvalue"]["mean_attempts"], 4)
     out["learned_vs_plain"] = rel_errors(mech, res["learned"], res["plain_kpphvalue"])
-    if args.tight_sample > 0:
+    from oracle import ref
+    if args.tight_sample > 0 and ref.available():
         nv = mech.nvar
         d = (np.abs(res["learned"][:nv] - res["plain_kpphvalue"][:nv]) /
              (mech.atol()[:, None] + mech.rtol()[:, None] * np.abs(res["plain_kpphvalue"][:nv]))).max(axis=0)
