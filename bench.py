@@ -12,8 +12,8 @@ Two legs on the same inputs:
   plain    one lane per cell (k_integrate), Hstart = 1e-5 s (cold start)
   learned  the MLP predicts each cell's h0 and cost class (bf16 MFMA), the
            cells are ordered costliest first, and the persistent solver
-           (k_persist, autotuned) integrates them; prediction and ordering
-           are inside the timed region.
+           (k_wave or k_persist, autotuned) integrates them; prediction and
+           ordering are inside the timed region.
 value = learned-leg cells/s; the plain leg is reported beside it.
 
 Other workloads (--workload): mixed (144x91x72, fullchem/Hg/carbon
@@ -88,6 +88,40 @@ def copy_calibration():
         y.copy_(x)
     torch.cuda.synchronize()
     print(json.dumps({"copy_calibration_bytes": 1 << 30, "repeats": 5}), flush=True)
+
+
+def dominant_kernel(cfg, integrate_ms, ho):
+    """(kernel, its ms, attempts of the other launch) of a persistent solve with
+    configuration cfg (Context.persistent_config) whose Integrate took
+    integrate_ms.  ho: Context.handoff_stats of the solve, or None; its lane
+    launch is the kernel when cells were handed off, and the attempts of the
+    cell-per-wave launch that followed are not its own.  Without a hand-off
+    (variant 7 has none) the solve is one launch."""
+    if cfg["wave_per_cell"]:
+        return "k_wave (one wavefront per cell, variant %d)" % cfg["variant"], integrate_ms, 0
+    name = "k_persist (one lane per cell, variant %d)" % cfg["variant"]
+    if ho is not None and ho[2] > 0:
+        return name, float(ho[2]), ho[1]
+    return name, integrate_ms, 0
+
+
+def handoff_report(max_cells, ho, integrate_ms):
+    """The hand-off's entry of the result line; None when none took place."""
+    if ho is None or not ho[2] > 0:
+        return None
+    return {"max_cells": max_cells, "cells_handed_off": int(round(ho[0])),
+            "cell_per_wave_attempts": int(round(ho[1])), "lane_launch_ms": round(float(ho[2]), 3),
+            "cell_per_wave_launch_ms": round(float(ho[3]), 3), "integrate_ms": round(integrate_ms, 3)}
+
+
+def split_report(cfg, split):
+    """How the warm learned step was launched."""
+    if split <= 0:
+        return "one persistent kernel, class order"
+    if cfg["wave_per_cell"]:
+        return "cells ordered by learned h0, smallest first; one cell-per-wave kernel"
+    return ("cells ordered by learned h0, smallest first; the first %d of a launch on the "
+            "cell-per-wave kernel beside the lane kernel" % split)
 
 
 def log(msg):
@@ -312,8 +346,9 @@ def grid_bench(args):
             tim.append(ctx.step_timings())
             if name == "learned" and args.handoff > 0:
                 hos.append(ctx.handoff_stats())
-                log("hand-off: %d cells, %d attempts; lane launch %.1f ms, cell-per-wave launch "
-                    "%.1f ms" % hos[-1])
+                if hos[-1][2] > 0:
+                    log("hand-off: %d cells, %d attempts; lane launch %.1f ms, cell-per-wave launch "
+                        "%.1f ms" % hos[-1])
             log("%s step done: %.1f ms total, integrate %.1f ms" % (name, tim[-1][3], tim[-1][1]))
         torch.cuda.synchronize()
         wall = time.perf_counter() - t0
@@ -326,22 +361,16 @@ def grid_bench(args):
     e2e = end_to_end(args, w, ctx, ic, rc)
     warm = None if args.no_warm else warm_legs(args, mech, w, ctx, model, P, ic, rc)
 
-    # dominant kernel: the persistent integrate (k_persist) of the learned
-    # leg; with the hand-off, its own launch (HIP events around it) and its
-    # own attempts (all attempts less those of the cell-per-wave launch,
-    # counted at the first-attempt cost: rejections are 0.3 % of attempts)
+    # dominant kernel: the integrate kernel of the learned leg; with a
+    # hand-off its own launch (HIP events around it) and its own attempts (all
+    # less those of the cell-per-wave launch, counted at the first-attempt
+    # cost: rejections are 0.3 % of attempts)
     nacc, nstp = L["st"][3].astype(np.int64), L["st"][2].astype(np.int64)
-    flop = FLOP_ACC * nacc.sum() + FLOP_REJ * (nstp - nacc).sum()
-    k_ms = float(np.mean([t[1] for t in L["tim"]]))
-    handoff = None
-    if L["hos"]:
-        ho = np.array(L["hos"], dtype=np.float64).mean(axis=0)
-        flop -= FLOP_ACC * ho[1]
-        k_ms = float(ho[2])
-        handoff = {"max_cells": args.handoff, "cells_handed_off": int(round(ho[0])),
-                   "cell_per_wave_attempts": int(round(ho[1])), "lane_launch_ms": round(ho[2], 3),
-                   "cell_per_wave_launch_ms": round(ho[3], 3),
-                   "integrate_ms": round(float(np.mean([t[1] for t in L["tim"]])), 3)}
+    int_ms = float(np.mean([t[1] for t in L["tim"]]))
+    ho = np.array(L["hos"], dtype=np.float64).mean(axis=0) if L["hos"] else None
+    kernel, k_ms, away = dominant_kernel(pcfg, int_ms, ho)
+    handoff = handoff_report(args.handoff, ho, int_ms)
+    flop = FLOP_ACC * (nacc.sum() - away) + FLOP_REJ * (nstp - nacc).sum()
     achieved = flop / (k_ms * 1e-3) / 1e12
     # HBM bytes per launch from the committed rocprof pass (FETCH_SIZE and
     # WRITE_SIZE, copy-calibrated), when it measured this variant on this grid
@@ -408,8 +437,8 @@ def grid_bench(args):
         "roofline": {"bound": "fp64_valu", "achieved": round(achieved, 4), "peak": PEAK_FP64_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP64_TFLOPS, 6),
                      "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": "k_persist (persistent Rodas3, FP64 sparse; the algorithmic work "
-                               "per attempt from the mechanism tables)",
+                     "kernel": kernel + ": persistent Rodas3, FP64 sparse; the algorithmic work "
+                               "per attempt from the mechanism tables",
                      "kernel_ms": round(k_ms, 3),
                      "hbm_TBps": None if traffic is None else round(traffic / (k_ms * 1e-3) / 1e12, 3),
                      "hbm_frac": None if traffic is None else round(traffic / (k_ms * 1e-3) / 1e12 / PEAK_HBM_TBPS, 4)},
@@ -563,9 +592,7 @@ def warm_legs(args, mech, w, ctx, model, P, ic, rc):
     out["workload"] = ("the step after the timed step: its plain-leg result perturbed by synthetic "
                        "emissions (NO, CO, ISOP, CH2O, SO2, ALD2 in P > 700 hPa) and 5% transport "
                        "noise, sun 20 min later, Hstart = KPPHvalue (reference) or learned h0")
-    out["learned_split"] = ("cells ordered by learned h0, smallest first; the first %d on the "
-                            "cell-per-wave kernel beside the lane kernel" % args.split
-                            if args.split > 0 else "one persistent kernel, class order")
+    out["learned_split"] = split_report(ctx.persistent_config(), args.split)
     out["handoff_max_cells"] = args.handoff
     return out
 
@@ -670,7 +697,8 @@ def mixed_bench(args):
     # the first replayed step (cold, Hstart 0) against the compiled reference
     # on the same cells, per mechanism
     accuracy, parity = {}, {}
-    if args.cpu_sample > 0:
+    from oracle import ref
+    if args.cpu_sample > 0 and ref.available():
         for m, p, ix, c in zip(mechs, parts, sample, first):
             ic, rc = icntrl_for(m.name)
             cref = reference_step(m, p.subset(ix), ic, rc, hstart=np.zeros(len(ix)))
@@ -881,17 +909,15 @@ def c90_bench(args):
     flop = 0.0
     for (_, _, nacc, ntot, _) in res[("learned", False)][4]:
         flop += FLOP_ACC * nacc + FLOP_REJ * (ntot - nacc)
-    kms = res[("learned", False)][1]
     ho = res[("learned", False)][5]
-    if args.handoff > 0:   # k_persist's own launches and attempts (see grid_bench)
-        flop -= FLOP_ACC * ho[1]
-        kms = ho[2]
+    pc = ctx.persistent_config()
+    kernel, kms, away = dominant_kernel(pc, res[("learned", False)][1], ho)  # as in grid_bench
+    flop -= FLOP_ACC * away
     achieved = flop / (kms * 1e-3) / 1e12
     # HBM bytes per chunk launch from the committed rocprof passes over this
     # workload (FETCH_SIZE and WRITE_SIZE, copy-calibrated, the mean of the
     # six lane launches), when they measured this configuration
     traffic = None
-    pc = ctx.persistent_config()
     traffic_src = ("no committed rocprof pass for variant %d, %d waves, hand-off %d"
                    % (pc["variant"], pc["waves"], args.handoff))
     tfile = ROOT / "profiles" / "persist_traffic.json"
@@ -916,20 +942,15 @@ def c90_bench(args):
                        "persistent_config": ctx.persistent_config(),
                        "wave_cap_first_face_cold_ms": {str(k): round(v, 1) for k, v in cap_ms.items()},
                        "handoff_max_cells": args.handoff},
-            "handoff_cold": None if args.handoff <= 0 else {
-                "cells_handed_off": ho[0], "cell_per_wave_attempts": ho[1],
-                "lane_launch_ms": round(ho[2], 3), "cell_per_wave_launch_ms": round(ho[3], 3)},
+            "handoff_cold": handoff_report(args.handoff, ho, res[("learned", False)][1]),
             "learned": L, "plain_gpu": P, "speedup_vs_plain": round(P["ms_per_step"] / L["ms_per_step"], 3),
             "warm_step": {"learned": Lw, "plain_kpphvalue": Pw,
                           "speedup_vs_plain": round(Pw["ms_per_step"] / Lw["ms_per_step"], 3),
-                          "learned_split": ("cells ordered by learned h0, smallest first; the first "
-                                            "%d of each chunk on the cell-per-wave kernel beside "
-                                            "the lane kernel" % args.split
-                                            if args.split > 0 else "one persistent kernel")},
+                          "learned_split": split_report(pc, args.split)},
             "roofline": {"bound": "fp64_valu", "achieved": round(achieved, 4), "peak": PEAK_FP64_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP64_TFLOPS, 6), "traffic": traffic,
                          "traffic_source": traffic_src,
-                         "kernel": "k_persist over the six chunks of the cold step (traffic: per chunk launch)",
+                         "kernel": kernel + " over the six chunks of the cold step (traffic: per chunk launch)",
                          "kernel_ms": round(kms, 3),
                          "hbm_TBps": None if hbm is None else round(hbm, 3),
                          "hbm_frac": None if hbm is None else round(hbm / PEAK_HBM_TBPS, 4)},
