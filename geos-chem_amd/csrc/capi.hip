@@ -69,7 +69,7 @@ struct gckpp_ctx {
   float *hlog;         // persistent solver: step-history log (device), or null
   int hlog_n;
   int pvariant;        // persistent kernel variant (loads in flight x register budget)
-  bool pchosen;        // by the caller (gckpp_set_persistent_config, the autotuner)
+  bool pchosen;        // by the caller (gckpp_set_persistent_config)
   int pwpb;            // waves per workgroup of the persistent launch
   int64_t pwaves;      // waves of one persistent launch (multiple of pwpb)
   int64_t pwaves_max;  // caller's cap on pwaves (0: every resident wave)
@@ -409,9 +409,9 @@ static void fill_persist_queue(const gckpp_ctx *c, IntegrateArgs &a, int64_t nce
 // waits for both.  With a hand-off set (lane variants), the lane kernel's
 // last unfinished cells move at a step boundary to a cell-per-wave launch
 // that follows it on s.  Neither for the unrolled lane kernel (Hg) unless the
-// caller chose its configuration: a cell-per-wave launch has one cell a wave
-// where this one has 64, and the hand-off's list of 98,304 cells took
-// 27 ms of a 50 ms grid step.
+// caller chose its configuration (gckpp_set_persistent_config): a
+// cell-per-wave launch has one cell a wave where this one has 64, and the
+// hand-off's list of 98,304 cells took 27 ms of a 50 ms grid step.
 static int launch_persist_queue(gckpp_ctx *c, PersistArgs &pa, int64_t ncell, hipStream_t s,
                                 const char *who) {
   const bool whole = unrolled_kernel(c->mech) && !c->pchosen;
@@ -1279,7 +1279,12 @@ extern "C" int gckpp_persistent_variants(void) { return PERSIST_VARIANTS; }
 // Times the persistent solver on the caller's cells for every variant and
 // workgroup size, keeps the fastest, and leaves conc untouched (each trial
 // integrates a copy).  ms[v*3 + g] receives the time of variant v with
-// 2^g waves per workgroup (-1 where it does not fit).
+// 2^g waves per workgroup (-1 where it does not fit).  A trial runs under the
+// context's split and hand-off as a later solve does: the tuner leaves pchosen
+// alone, so that neither comes into force with its choice (for Hg it did, and a
+// hand-off that no trial had run took 27 ms of every 50 ms grid step).  Where
+// every lane variant is one kernel (unrolled_kernel) that kernel is timed
+// once and its time stands for them all.
 extern "C" int gckpp_autotune_dev(gckpp_ctx *c, int64_t ncell, double tin, double tout,
                                   const int32_t icntrl[20], const double rcntrl[20],
                                   const double *hstart, const double *conc,
@@ -1293,13 +1298,17 @@ extern "C" int gckpp_autotune_dev(gckpp_ctx *c, int64_t ncell, double tin, doubl
   const size_t cbytes = sizeof(double) * c->info.nspec * ncell;
   int32_t *ierr = (int32_t *)(scratch + (size_t)c->info.nspec * ncell);
   int keep_solver = c->solver, best_v = c->pvariant, best_g = c->pwpb;
-  float best = -1.0f;
+  float best = -1.0f, lane = -1.0f;
   c->solver = GCKPP_SOLVER_PERSISTENT;
   int rc = 0;
   for (int v = 0; v < PERSIST_VARIANTS && rc == 0; ++v) {
     for (int g = 0; g < 3 && rc == 0; ++g) {
       float t = -1.0f;
-      if (set_pconfig(c, v, 1 << g) == 0) {
+      const bool fits = set_pconfig(c, v, 1 << g) == 0;
+      const bool unrolled = unrolled_kernel(c->mech) && v != PERSIST_WAVE_VARIANT;
+      if (fits && unrolled && lane >= 0.0f) {
+        t = lane;
+      } else if (fits) {
         // one untimed run of the first configuration warms caches and code
         for (int rep = (v == 0 && g == 0) ? 0 : 1; rep < 2 && rc == 0; ++rep) {
           HIP_OK(hipMemcpyAsync(scratch, conc, cbytes, hipMemcpyDeviceToDevice, s));
@@ -1315,12 +1324,12 @@ extern "C" int gckpp_autotune_dev(gckpp_ctx *c, int64_t ncell, double tin, doubl
           best_v = v;
           best_g = 1 << g;
         }
+        if (unrolled) lane = t;
       }
       if (ms) ms[v * 3 + g] = t;
     }
   }
   c->solver = keep_solver;
-  c->pchosen = true;
   if (set_pconfig(c, best_v, best_g) != 0) set_pconfig(c, kDefaultLaneVariant, 1);
   return rc;
 }

@@ -367,8 +367,10 @@ int gckpp_persistent_handoff_stats(gckpp_ctx *ctx, int64_t n[2], float ms[2]);
 
 /* Autotuner: integrates a copy of the given cells with every persistent
  * configuration, keeps the fastest for this context and writes the times
- * [ms] to ms[variant*3 + log2(waves_per_group)] (-1: does not fit).  conc is
- * not modified.  Synchronous on stream. */
+ * [ms] to ms[variant*3 + log2(waves_per_group)] (-1: does not fit).  The
+ * trials run under the context's split and hand-off as a later solve does.
+ * Hg's lane variants are one kernel: it is timed once, and its time written
+ * for each of them.  conc is not modified.  Synchronous on stream. */
 int gckpp_autotune_dev(gckpp_ctx *ctx, int64_t ncell, double tin, double tout,
                        const int32_t icntrl[20], const double rcntrl[20],
                        const double *hstart, const double *conc,
