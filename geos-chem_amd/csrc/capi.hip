@@ -1465,8 +1465,8 @@ static int batch_enqueue(gckpp_batch *b, const gckpp_part parts[3], double dt, h
   pa.slot_fields = launch_slot_fields(PQ_MIXED, variant);
   pa.counter = b->counter;
   const bool hand = b->ho_cap > 0 && b->ho_rec && variant != PERSIST_WAVE_VARIANT;
+  if (b->ho_ctr) launch_zero_u32(b->ho_ctr, 4, s);  // (the count of a step without one is 0)
   if (hand) {
-    launch_zero_u32(b->ho_ctr, 4, s);
     pa.ho = Handoff{b->ho_ctr, b->ho_ctr + 1, b->ho_ctr + 3, b->ho_cell, b->ho_rec, b->ho_cap, 0};
   }
   int64_t nw = cells_to_waves(variant, end);
@@ -1524,7 +1524,10 @@ extern "C" int gckpp_batch_set_handoff(gckpp_batch *b, int64_t max_cells) {
     hipError_t e = hipMalloc(&b->ho_cell, sizeof(int32_t) * (size_t)max_cells);
     if (e == hipSuccess)
       e = hipMalloc(&b->ho_rec, sizeof(double) * (size_t)(HO_FIELDS + nvar) * (size_t)max_cells);
-    if (e == hipSuccess && !b->ho_ctr) e = hipMalloc(&b->ho_ctr, 4 * sizeof(unsigned int));
+    if (e == hipSuccess && !b->ho_ctr) {
+      e = hipMalloc(&b->ho_ctr, 4 * sizeof(unsigned int));
+      if (e == hipSuccess) e = hipMemset(b->ho_ctr, 0, 4 * sizeof(unsigned int));
+    }
     if (e == hipSuccess && !b->hwork) {
       const int64_t res = persist_resident_waves(PQ_MIXED, PERSIST_WAVE_VARIANT, 1);
       if (res <= 0) e = hipErrorInvalidConfiguration;

@@ -74,3 +74,44 @@ def test_rates_do_not_depend_on_the_number_of_cells(n, inputs, fullchem, torch_d
                   _t(torch_dev, w.conc[:, :n])).cpu().numpy()
     ctx.close()
     assert np.array_equal(r, rct[:, :n])
+
+
+def test_handoff_count_is_the_last_steps(inputs, fullchem, hg, torch_dev):
+    """gckpp_batch_handoff_count after a step that handed cells over, then after
+    steps that did not: eager, and replayed from a graph."""
+    from gckpp_amd import hip, synth
+    print("case: hand-off count of a batch", flush=True)
+    T = torch_dev
+    mechs = [fullchem, hg]
+    ws = [synth.box_cells(m, 256, 3) for m in mechs]
+    ctxs = [hip.Context(m, w.ncell) for m, w in zip(mechs, ws)]
+    B = hip.Batch(*ctxs)
+    st = [dict(met=_t(T, w.met), photol=_t(T, w.photol), het=_t(T, w.het), conc=_t(T, w.conc),
+               hstart=_t(T, np.zeros(w.ncell)), icntrl=options.icntrl_for(m.name)[0],
+               rcntrl=options.icntrl_for(m.name)[1],
+               istatus=T.zeros((20, w.ncell), dtype=T.int32, device="cuda"),
+               ierr=T.zeros(w.ncell, dtype=T.int32, device="cuda")) for m, w in zip(mechs, ws)]
+    parts = [B.part(**d) for d in st]
+
+    def count(variant, replay):
+        B.set_config(variant, 1)
+        if replay:
+            B.capture(parts, 1200.0)
+            B.replay()
+        else:
+            B.step(parts, 1200.0)
+        T.cuda.synchronize()
+        return B.handoff_count()
+
+    B.set_handoff(100)
+    assert B.handoff_count() == 0            # no step yet
+    assert count(4, False) > 0
+    assert count(hip.WAVE_VARIANT, False) == 0
+    assert count(4, True) > 0
+    assert count(hip.WAVE_VARIANT, True) == 0
+    assert count(4, False) > 0
+    B.set_handoff(0)
+    assert count(4, False) == 0
+    B.close()
+    for c in ctxs:
+        c.close()
