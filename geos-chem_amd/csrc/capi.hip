@@ -1417,6 +1417,26 @@ extern "C" int gckpp_batch_init(gckpp_ctx *fullchem, gckpp_ctx *hg, gckpp_ctx *c
   return 0;
 }
 
+// The kernel of a batch without a configuration of the caller's that has nf
+// fullchem and nh Hg cells of total: true for the lane kernel (with the hand-off
+// of cap cells where one is set), false for the cell-per-wave kernel.  Both
+// times as estimated from cold steps of 100 to 100,000 fullchem and 30,000 to
+// 500,000 Hg cells, in microseconds.  A fullchem cell takes 2.6 on a wave of its
+// own (768 at a time), an Hg cell 1.17 there and 0.1 on a lane.  The lane
+// kernel's length is its longest fullchem chain, 560 ms and 6 more a cell; with
+// a hand-off its fullchem cells move on as soon as at most cap cells are left
+// (50 ms and 2.6 a cell), unless they alone are more than that (7.4 a cell).
+// Up to cap cells the hand-off takes every cell at once.  Measured, ms, wave /
+// lane and hand-off / lane: 10,000 + 30,000 cells 62 / 64 / -, 100 + 100,000 118
+// / 63 / -, 10,000 + 200,000 261 / 81 / 777, 30,000 + 500,000 667 / 191 / 909,
+// 100,000 + 200,000 503 / 787 / -; 14,008 + 4,002 (and 2,001 carbon) 42 / 43 / 766.
+static bool batch_on_lanes(int64_t nf, int64_t nh, int64_t total, int64_t cap) {
+  const double wave = 2.6 * nf + 1.17 * nh;
+  if (cap <= 0) return 560e3 + 6.0 * nf + 0.1 * nh < wave;
+  if (total <= cap) return false;
+  return 50e3 + (nf < cap ? 2.6 : 7.4) * nf + 0.1 * nh < wave;
+}
+
 // One part of a batch step: the cells of one mechanism (see gckpp_hip.h).
 static int batch_enqueue(gckpp_batch *b, const gckpp_part parts[3], double dt, hipStream_t s) {
   PersistArgs pa{};
@@ -1449,13 +1469,12 @@ static int batch_enqueue(gckpp_batch *b, const gckpp_part parts[3], double dt, h
     pa.qend[q] = end;
   }
   if (end == 0) return 0;
-  // Without a configuration of the caller's: the cell-per-wave kernel when the
-  // batch has fullchem cells, which then are nearly all of its work (20,011
-  // cells, 70/20/10 %: 50 ms where the lane kernel with the hand-off took
-  // 197 ms), else the lane kernel (64 Hg cells a wave).
+  // without a configuration of the caller's: the faster kernel for these
+  // counts; without fullchem cells the lane kernel (64 cells a wave)
   int variant = b->variant, wpb = b->wpb;
   int64_t nwaves = b->nwaves;
-  if (!b->chosen && pa.qend[0] > 0) {
+  if (!b->chosen && pa.qend[0] > 0 &&
+      !batch_on_lanes(pa.qend[0], pa.qend[1] - pa.qend[0], end, b->ho_rec ? b->ho_cap : 0)) {
     variant = PERSIST_WAVE_VARIANT;
     wpb = 1;
     nwaves = b->wave_waves;

@@ -401,7 +401,10 @@ typedef struct {
   const int32_t *order;       /* [ncell] order in which cells are taken, or null */
 } gckpp_part;
 /* contexts in the order fullchem, Hg, carbon; any may be null; each part's
- * ncell must not exceed its context's max_cells. */
+ * ncell must not exceed its context's max_cells.  Until gckpp_batch_set_config
+ * each step picks its kernel by its cells: the cell-per-wave kernel (variant 7)
+ * for fullchem cells, unless Hg cells are so many that the lane kernel is
+ * estimated to be faster; the lane kernel (variant 4) without fullchem cells. */
 int gckpp_batch_init(gckpp_ctx *fullchem, gckpp_ctx *hg, gckpp_ctx *carbon,
                      gckpp_batch **out);
 int gckpp_batch_set_config(gckpp_batch *b, int variant, int waves_per_group);
@@ -411,8 +414,8 @@ int gckpp_batch_set_config(gckpp_batch *b, int variant, int waves_per_group);
  * captured with. */
 int gckpp_batch_set_waves(gckpp_batch *b, int64_t max_waves);
 /* The tail hand-off of gckpp_set_persistent_handoff for the batch's launch
- * (fullchem and Hg cells; carbon cells finish on their lanes), captured
- * with the step; gckpp_batch_handoff_count: cells the last step handed
+ * (fullchem and Hg cells; carbon cells finish on their lanes; no effect on a
+ * step of the cell-per-wave kernel), captured with the step; gckpp_batch_handoff_count: cells the last step handed
  * over (synchronises the device).  A captured graph keeps the setting it
  * was captured with.  A max_cells larger than any before reallocates the
  * list: the call then waits for the device and destroys the captured

@@ -115,3 +115,60 @@ def test_handoff_count_is_the_last_steps(inputs, fullchem, hg, torch_dev):
     B.close()
     for c in ctxs:
         c.close()
+
+
+@pytest.mark.parametrize("counts,handoff,lanes", [((100, 60000, 10), 2000, True),      # Hg is the work
+                                                  ((100, 60000, 10), 0, False),        # ... no hand-off
+                                                  ((100, 60000, 10), 70000, False),    # ... of every cell
+                                                  ((5000, 60000, 10), 2000, False),    # fullchem over the cap
+                                                  ((700, 200, 100), 500, False)])
+def test_batch_picks_its_kernel_by_its_cells(counts, handoff, lanes, inputs, fullchem, hg, mech_of, torch_dev):
+    """A batch without a configuration: the lane kernel (then cells are handed
+    off) where many Hg cells stand beside few fullchem ones, the cell-per-wave
+    kernel otherwise; the results are those of the configured cell-per-wave
+    kernel, bit by bit, also replayed from a graph."""
+    from gckpp_amd import hip, synth
+    print("case: batch of %s cells, hand-off %d" % (counts, handoff), flush=True)
+    T = torch_dev
+    mechs = [fullchem, hg, mech_of("carbon")]
+    ws = [synth.box_cells(m, 1024, 3) for m in mechs]
+    ctxs = [hip.Context(m, n) for m, n in zip(mechs, counts)]
+    B = hip.Batch(*ctxs)
+
+    def state():
+        st = []
+        for m, w, n in zip(mechs, ws, counts):
+            ic, rc = options.icntrl_for(m.name)
+            i = np.arange(n) % w.ncell
+            het = w.het if w.het.shape[1] == 1 else w.het[:, i]
+            st.append(dict(met=_t(T, w.met[:, i]), photol=_t(T, w.photol[:, i]), het=_t(T, het),
+                           conc=_t(T, w.conc[:, i]), hstart=_t(T, np.zeros(n)), icntrl=ic, rcntrl=rc,
+                           istatus=T.zeros((20, n), dtype=T.int32, device="cuda"),
+                           ierr=T.zeros(n, dtype=T.int32, device="cuda")))
+        return st
+
+    def result(st):
+        T.cuda.synchronize()
+        return [d[k].cpu().numpy() for d in st for k in ("conc", "hstart", "istatus", "ierr")]
+
+    B.set_handoff(handoff)
+    st = state()
+    B.step([B.part(**d) for d in st], 1200.0)
+    a = result(st)
+    if handoff:
+        assert (B.handoff_count() > 0) == lanes
+    else:
+        assert B.handoff_count() == 0 and not lanes
+    sg = state()
+    pg = [B.part(**d) for d in sg]
+    B.capture(pg, 1200.0)
+    B.replay()
+    g = result(sg)
+    B.set_config(hip.WAVE_VARIANT, 1)
+    sw = state()
+    B.step([B.part(**d) for d in sw], 1200.0)
+    for x, y, z in zip(a, g, result(sw)):
+        assert np.array_equal(x, y) and np.array_equal(x, z)
+    B.close()
+    for c in ctxs:
+        c.close()
