@@ -103,6 +103,11 @@ template <> struct CellProg<Traits_fullchem> {
                                                double yd) {
     cell_fullchem::cell_solve(c, T, ud, yd);
   }
+  // the same with no read of an LU position that is not the sum's own
+  static __device__ __forceinline__ void solve_apart(const CellLds &c, const double (&T)[TAIL],
+                                                     double ud, double yd) {
+    cell_fullchem::cell_solve_apart(c, T, ud, yd);
+  }
   static __device__ __forceinline__ __amdgpu_buffer_rsrc_t words() {
     return brsrc(cell_fullchem::words, (int)sizeof(cell_fullchem::words));
   }
@@ -181,10 +186,18 @@ __device__ __forceinline__ void cell_finish(const IntegrateArgs &a, const CellLd
 }
 
 // One Rodas3 attempt of the wave's cell (lane_attempt's algorithm and order
-// of operations); true when the cell is done (S.ierr then holds IERR).
-template <class M>
-__device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellLds &c, int64_t cell,
-                                             RosState &S, CellState<M> &cs) {
+// of operations): CELL_DONE when the cell is done (S.ierr then holds IERR),
+// CELL_AGAIN when it has to be made again with APART.  P::solve lets a lane
+// whose terms have ended read another row's factor times 0, which an infinite
+// factor turns into a NaN of a row that has nothing to do with it.  A stage
+// vector's NaN reaches the error norm; so an attempt whose norm is NaN is made
+// again with P::solve_apart, and a row is NaN only where its own terms make it
+// so.  (As a second copy of the attempt: a branch around the solve costs every
+// attempt 1 %, its first loads no longer start before it.)
+enum { CELL_MORE = 0, CELL_DONE = 1, CELL_AGAIN = 2 };
+template <class M, bool APART>
+__device__ __forceinline__ int cell_attempt(const IntegrateArgs &a, const CellLds &c, int64_t cell,
+                                            RosState &S, CellState<M> &cs) {
   using P = CellProg<M>;
   constexpr int N = M::NVAR, KS = CellState<M>::KS;
   const RosParams &prm = a.prm;
@@ -204,7 +217,7 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
       v[k] = 64 * (k + 1) <= N || c.lane + 64 * k < N ? LDL(8 * (P::X0 + 64 * k)) : 0.0;
     wave_sync();
   };
-  if (S.newStep && state_done(prm, S)) return true;
+  if (!APART && S.newStep && state_done(prm, S)) return CELL_DONE;
   double K0[KS], K1[KS], K2[KS], K3[KS], T[P::TAIL], ud = 1.0, yd = 1.0, dH = 0.0;
 #pragma unroll
   for (int k = 0; k < KS; ++k) K0[k] = K1[k] = K2[k] = K3[k] = 0.0;
@@ -213,7 +226,7 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
   // s = -1: Fcn0 of a new step; s = 0: the matrix and its LU; s = 0..3: the
   // stages.  A loop, so that the programs are inlined once.
 #pragma unroll 1
-  for (int s = S.newStep ? -1 : 0; s < 4; ++s) {
+  for (int s = !APART && S.newStep ? -1 : 0; s < 4; ++s) {
     double v[KS];
     if (s < 0 || s >= 2) {
 #pragma unroll
@@ -252,7 +265,7 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
             else break;
           }
         }
-        if (singular) { S.ierr = -8; return true; }
+        if (singular) { S.ierr = -8; return CELL_DONE; }
         dH = dir * S.H;
       }
 #pragma unroll
@@ -268,7 +281,8 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
       }
     }
     put(v);
-    P::solve(c, T, ud, yd);
+    if constexpr (APART) P::solve_apart(c, T, ud, yd);
+    else P::solve(c, T, ud, yd);
     get(v);
     S.st[6] += 1;
 #pragma unroll
@@ -309,6 +323,12 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
 #pragma unroll
     for (int u = 0; u < 16; ++u) err += q[u];
   }
+  if (!APART && __any(err != err)) {
+    S.st[0] -= 2;  // (counted again: the stages' Fun, the LU, the substitutions)
+    S.st[5] -= 1;
+    S.st[6] -= 4;
+    return CELL_AGAIN;
+  }
   err = max_f(sqrt(err / N), 1.0e-10);
   if (a.hlog && S.st[2] < a.hlog_n && c.lane == 0) {
     a.hlog[(int64_t)(2 * S.st[2]) * a.ncell + cell] = (float)H;
@@ -318,7 +338,7 @@ __device__ __forceinline__ bool cell_attempt(const IntegrateArgs &a, const CellL
 #pragma unroll
     for (int k = 0; k < KS; ++k) cs.Y[k] = prm.clip_negative ? max_f(yn[k], 0.0) : yn[k];
   }
-  return false;
+  return CELL_MORE;
 }
 
 #undef LD

@@ -747,7 +747,9 @@ __global__ __launch_bounds__((64 * QueueLds<M0, M1, M2>::WPB), 1) void k_wave(Pe
     on_queue_w<M0, M1, M2>(q, [&](auto *tag) {
       using M = std::remove_pointer_t<decltype(tag)>;
       if constexpr (HasCell<M>::value) {
-        done = cell_attempt<M>(pa.q[q], cl, cell, S, cs);
+        int r = cell_attempt<M, false>(pa.q[q], cl, cell, S, cs);
+        if (r == CELL_AGAIN) r = cell_attempt<M, true>(pa.q[q], cl, cell, S, cs);
+        done = r == CELL_DONE;
       } else if constexpr (IsEulerW<M>::value) {
         wave_euler<M>(pa.q[q], WaveCell<M>{sh, g, lane}, S);
         done = true;

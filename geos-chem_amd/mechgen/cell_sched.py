@@ -509,10 +509,25 @@ class Stream:
         return out, flat
 
 
-def emit_rounds(st, rounds, kind, L, tag):
+def side_by_side(rd, x, L):
+    """The first LU position of step x of a round of kind 'n' when the step's
+    factors lie side by side, lane by lane (see solve_order); else None."""
+    fs = [p.terms[x][0] for p in rd.pieces if x < len(p.terms)]
+    if fs[-1] < L["LUH"] and fs == list(range(fs[0], fs[0] + len(fs))) and \
+            all(x < len(p.terms) for p in rd.pieces[:len(fs)]):
+        return fs[0]
+    return None
+
+
+def emit_rounds(st, rounds, kind, L, tag, own=True):
     """A phase's rounds: the operands of up to DEPTH steps are requested ahead,
     across round ends too, but never before the stores of the round they wait
-    for (LDS operations of a wave execute in order, so no wait is needed)."""
+    for (LDS operations of a wave execute in order, so no wait is needed).
+    own: steps whose factors lie side by side read them at a fixed offset from
+    the lane's own slot.  A lane whose terms have ended then reads the LU
+    position after the step's factors, times 0: harmless unless that position
+    is infinite or NaN, which makes the lane's sum NaN.  Without own every idle
+    lane reads the zero slot."""
     zero, one, sink = L["ZERO"], L["ONE"], L["SINK"]
     pad = (zero, 0 if kind != "n" else zero)
     seq = []
@@ -542,14 +557,13 @@ def emit_rounds(st, rounds, kind, L, tag):
                 st.line("const double d%s = LD(%s);" % (n, st.word(d)))
         elif k == "T":
             w = []
-            fs = [p.terms[x][0] for p in rd.pieces if x < len(p.terms)]
-            if kind == "n" and fs[-1] < L["LUH"] and fs == list(range(fs[0], fs[0] + len(fs))) and \
-                    all(x < len(p.terms) for p in rd.pieces[:len(fs)]):
+            f = side_by_side(rd, x, L) if own and kind == "n" else None
+            if f is not None:
                 for ln in range(LANES):
-                    t = rd.pieces[ln].terms if ln < len(fs) else []
-                    w.append(8 * (t[x][1] if t else zero))
+                    t = rd.pieces[ln].terms if ln < len(rd.pieces) else []
+                    w.append(8 * (t[x][1] if x < len(t) else zero))
                 st.line("const double a%s_%d = LDL(%d), b%s_%d = LD%s;"
-                        % (n, x, 8 * fs[0], n, x, st.half(w)))
+                        % (n, x, 8 * f, n, x, st.half(w)))
                 return
             for ln in range(LANES):
                 t = rd.pieces[ln].terms if ln < len(rd.pieces) else []
@@ -683,10 +697,8 @@ def emit_code(m, t, o):
         st.line("} }")
     st.line("yd = 1.0 / ud;")
     func("cell_lu", ", double (&T)[%d], double &ud, double &yd" % k, st)
-    # substitutions: forward in front of the block, the block, backward
-    st = Stream("solve")
-    sched["sf"] = o["sf"].schedule()
-    emit_rounds(st, sched["sf"], "n", L, "f")
+    # substitutions of the block: x of the lane's row, in X before and after
+    st = Stream("tail")
     st.line("wave_sync();")
     st.line("double x = LDL(%d);" % (8 * (L["X"] + s)))
     st.line("x = c.lane < %d ? x : 0.0;" % k)
@@ -709,7 +721,15 @@ def emit_code(m, t, o):
     st.line("}")
     st.line("if (c.lane < %d) STL(%d, q);" % (k, 8 * (L["X"] + s)))
     st.line("wave_sync();")
-    sched["sb"] = o["sb"].schedule()
-    emit_rounds(st, sched["sb"], "n", L, "b")
-    func("cell_solve", ", const double (&T)[%d], double ud, double yd" % k, st)
+    args = ", const double (&T)[%d], double ud, double yd" % k
+    func("cell_tail", args, st)
+    # substitutions: forward in front of the block, the block, backward; and
+    # the same without a read of an unrelated LU position
+    sched["sf"], sched["sb"] = o["sf"].schedule(), o["sb"].schedule()
+    for name, own in (("cell_solve", True), ("cell_solve_apart", False)):
+        st = Stream("solve")
+        emit_rounds(st, sched["sf"], "n", L, "f", own)
+        st.line("cell_tail(c, T, ud, yd);")
+        emit_rounds(st, sched["sb"], "n", L, "b", own)
+        func(name, args, st)
     return "\n".join(out), all_words, sched

@@ -5,6 +5,7 @@ it) they give bit-identical Vdot, Jacobian, LU and substitution results on
 random data with the mechanism's pattern; no round reads what a later round,
 or one it was not told to wait for, writes; and every word's offsets stay
 inside the wave's LDS block and the coefficient table."""
+import re
 import sys
 from pathlib import Path
 
@@ -177,3 +178,125 @@ def test_generated_header_holds_the_programs(cell):
     i = hdr.index("unsigned words[%d]" % len(words))
     body = hdr[hdr.index("{", i) + 1:hdr.index("}", i)]
     assert [int(x) for x in body.split(",") if x.strip()] == words
+
+
+class Emitted:
+    """Runs the emitted code of one program on 64 lanes (one IEEE double
+    operation per statement and lane; no fused multiply-add, as in the walk it
+    is compared with), idle lanes included."""
+
+    def __init__(self, code, words, lds):
+        self.lds, self.words, self.v = lds, np.array(words, dtype=np.uint64).reshape(-1, 64, 4), {}
+        self.code, self.lane = code, np.arange(64)
+
+    def function(self, name):
+        body = self.code[self.code.index("void %s(" % name):]
+        body = body[body.index("{") + 1:body.index("#undef LDW")].split("\n")
+        base = int(body[1].split("cell_word(c, ")[1].split(" ")[0])
+        return base, [x.strip() for x in body[2:] if x.strip()]
+
+    def expr(self, e):
+        """A word, h >> 16, (w & 0xffffu), LD(...), LDL(k), 0.0, a name."""
+        e = e.strip()
+        if e.startswith("LDL("):
+            return self.lds[int(e[4:-1]) // 8 + self.lane]
+        if e.startswith("LD"):
+            return self.lds[self.expr(e[2:]).astype(np.int64) // 8]
+        if e.startswith("(") and e.endswith(")"):
+            return self.expr(e[1:-1])
+        if e.endswith(">> 16"):
+            return self.expr(e[:-5]) >> np.uint64(16)
+        if e.endswith("& 0xffffu"):
+            return self.expr(e[:-9]) & np.uint64(0xFFFF)
+        m = re.fullmatch(r"w(\d+)\.([xyzw])", e)
+        if m:
+            return self.words[self.base + int(m.group(1)), :, "xyzw".index(m.group(2))]
+        return np.zeros(64) if e == "0.0" else self.v[e]
+
+    def run(self, name, tail):
+        self.base, lines = self.function(name)
+        self.v = {}
+        for s in lines:
+            m = re.fullmatch(r"const double (a\w+) = (.*), (b\w+) = (.*);", s)
+            if m:
+                self.v[m.group(1)], self.v[m.group(3)] = self.expr(m.group(2)), self.expr(m.group(4))
+                continue
+            m = re.fullmatch(r"(c\w+) = fma\(-(\w+), (\w+), (\w+)\);", s)
+            if m:
+                c, a, b, c0 = (self.v.get(x) for x in m.groups())
+                self.v[m.group(1)] = c0 + (-a) * b
+                continue
+            m = re.fullmatch(r"ST\((h\w+) & 0xffffu, (c\w+)(?: / (d\w+))?\);", s)
+            if m:
+                v = self.v[m.group(2)] / self.v[m.group(3)] if m.group(3) else self.v[m.group(2)]
+                self.lds[(self.v[m.group(1)] & np.uint64(0xFFFF)).astype(np.int64) // 8] = v
+                continue
+            m = re.fullmatch(r"(?:const )?(?:unsigned|double) (\w+) = (.*);", s)
+            if m:
+                self.v[m.group(1)] = np.array(self.expr(m.group(2)))
+                continue
+            if s.startswith("cell_tail("):
+                tail(self.lds)
+            else:
+                assert s.startswith("const u32x4 w"), s
+
+
+def test_infinite_factors_reach_their_own_rows_only(cell):
+    """A lane whose terms have ended reads another row's factor times 0 in
+    cell_solve.  With finite factors it gives the walk's result; an infinite
+    one makes NaN of rows that have nothing to do with it, but every result
+    that differs from the walk's holds a NaN (the solver's sign to take
+    cell_solve_apart), and cell_solve_apart's never differs."""
+    C, raw, t, o, code, words, sched = cell
+    rng = np.random.default_rng(17)
+    nv, nz, s, k, L = raw["nvar"], raw["lu_nonzero"], o["s"], o["tail"], o["layout"]
+    crow, diag, icol, irow = (raw[x] for x in ("lu_crow", "lu_diag", "lu_icol", "lu_irow"))
+    lu0 = rng.uniform(-1.0, 1.0, nz) * 0.1
+    lu0[diag[:nv]] = rng.uniform(5.0, 9.0, nv)
+    x0 = rng.uniform(-1.0, 1.0, nv)
+    head = [q for q in range(nz) if o["lu"][q] < L["LUH"]]
+    spoiled = 0
+    with np.errstate(all="ignore"):
+        for bad in [None] + list(rng.choice(head, 40, replace=False)):
+            lu = lu0.copy()
+            if bad is not None:
+                lu[bad] = rng.choice([np.inf, -np.inf, np.nan])
+            x = list(x0)
+            sub = lambda acc, q: acc + (-lu[q]) * x[icol[q]]
+            for i in range(nv):
+                x[i] = chunked(C, x[i], list(range(crow[i], diag[i])), t["fw_hd"][i] - crow[i], sub)
+            y = list(x)
+            for i in range(nv - 1, -1, -1):
+                ks = list(range(crow[i + 1] - 1, diag[i], -1))
+                x[i] = chunked(C, x[i], ks, len(ks) if i < s else 0, sub) / lu[diag[i]]
+
+            def tail(lds, ref=(y, x)):   # the block's rows before and after
+                X = slice(L["X"] + s, L["X"] + nv)
+                z = lds[X].copy()
+                for j in range(k):
+                    for q in range(crow[s + j], diag[s + j]):
+                        if icol[q] >= s:
+                            z[j] = z[j] + (-lu[q]) * z[icol[q] - s]
+                for j in range(k - 1, -1, -1):
+                    for q in range(crow[s + j + 1] - 1, diag[s + j], -1):
+                        z[j] = z[j] + (-lu[q]) * z[icol[q] - s]
+                    z[j] = z[j] / lu[diag[s + j]]
+                lds[X] = z
+
+            got = {}
+            for name in ("cell_solve", "cell_solve_apart"):
+                lds = np.zeros(L["SIZE"])
+                lds[L["ONE"]], lds[L["NEG"]] = 1.0, -1.0
+                for q in range(nz):
+                    lds[o["lu"][q]] = lu[q]
+                lds[L["X"]:L["X"] + nv] = x0
+                e = Emitted(code, words, lds)
+                e.run(name, tail)
+                got[name] = lds[L["X"]:L["X"] + nv].copy()
+            assert np.array_equal(got["cell_solve_apart"], x, equal_nan=True)
+            if bad is None:
+                assert np.array_equal(got["cell_solve"], x) and np.isfinite(x).all()
+            elif not np.array_equal(got["cell_solve"], x, equal_nan=True):
+                assert np.isnan(got["cell_solve"]).any()
+                spoiled += int((np.isfinite(x) & np.isnan(got["cell_solve"])).any())
+    assert spoiled > 0    # (the case that cell_solve_apart is there for)

@@ -177,3 +177,41 @@ def test_batch_picks_its_kernel_by_its_cells(counts, handoff, lanes, inputs, ful
     B.close()
     for c in ctxs:
         c.close()
+
+
+@pytest.mark.parametrize("factor", [np.inf, 1.0e300])
+def test_infinite_entries_spoil_the_same_rows_in_every_kernel(factor, inputs, fullchem, torch_dev):
+    """One reaction a cell with a rate whose Jacobian entries overflow, for each
+    of the mechanism's reactions, and reactants at zero in every other cell: at
+    most two attempts, after which the cell-per-wave kernel holds NaN and
+    infinities exactly where the lane kernel does.  (Where unrelated rows of
+    the factorisation meet, a row that stays finite has to stay the same.)"""
+    from gckpp_amd import hip
+    print("case: one overflowing reaction a cell, rate times %g" % factor, flush=True)
+    m, n = fullchem, fullchem.nreact
+    _, conc, rct = inputs["fullchem"]
+    cells = (np.arange(n) * 37) % conc.shape[1]
+    c0, r = conc[:, cells].copy(), rct[:, cells].copy()
+    for k, rx in enumerate(m.reactions):
+        r[k, k] = max(r[k, k], 1.0e-20) * factor
+        if k % 2:
+            for sp, mult in rx["reactants"]:
+                if sp < m.nvar:
+                    c0[sp, k] = 0.0
+    ic, rc = options.fullchem_icntrl()
+    ic = ic.copy()
+    ic[3] = 1
+    out = []
+    for v in (7, 4):
+        ctx = hip.Context(m, n)
+        ctx.set_solver(hip.SOLVER_PERSISTENT)
+        ctx.set_persistent_config(v, 1)
+        c = _t(torch_dev, c0)
+        ist, rst, ierr = ctx.integrate(c, _t(torch_dev, r), _t(torch_dev, np.full(n, 1.0)), 0.0, 1200.0, ic, rc)
+        out.append([x.cpu().numpy() for x in (c, ist, rst, ierr)])
+        ctx.close()
+    some = np.isnan(out[0][0]).any(0) & np.isfinite(out[0][0][:m.nvar]).any(0)
+    print("cells with NaN and finite species: %d of %d" % (some.sum(), n))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
+    assert some.sum() > 20
