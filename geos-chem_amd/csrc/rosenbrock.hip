@@ -58,48 +58,41 @@ struct BCol {
 };
 
 // ---------------------------------------------------------------------------
-// acc + sum_{t0<=t<t1} w(t)*v(t), added in increasing t.  With U > 1 the
-// operands of U terms are loaded before their FMAs, so a wave keeps up to 2U
-// loads in flight instead of waiting on each term; the sum (and its rounding)
-// is the same for every U.
-template <int U, class W, class V>
-__device__ __forceinline__ double gather_fma(int t0, int t1, double acc, W w, V v) {
+// acc + sum_{t0<=t<t1} w(k)*v(k), added in increasing t; k = t, or, DOWN, the
+// table entries from last downwards: k = last - t.  With U > 1 the operands of
+// U terms are loaded before their FMAs, so a wave keeps up to 2U loads in
+// flight instead of waiting on each term; the sum (and its rounding) is the
+// same for every U.  (DOWN: a batch's entries as its lowest one plus a constant,
+// which the loads take as their immediate offsets.)
+template <int R, bool DOWN, class W, class V>
+__device__ __forceinline__ void gather_batch(int t, int last, double &acc, W w, V v) {
+  const int k = DOWN ? last - t - (R - 1) : t;
+  double a[R], b[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    a[u] = w(k + (DOWN ? R - 1 - u : u));
+    b[u] = v(k + (DOWN ? R - 1 - u : u));
+  }
+#pragma unroll
+  for (int u = 0; u < R; ++u) acc = fma(a[u], b[u], acc);
+}
+template <int U, bool DOWN = false, class W, class V>
+__device__ __forceinline__ double gather_fma(int t0, int t1, double acc, W w, V v, int last = 0) {
   int t = t0;
-  if constexpr (U >= 16) {
-    for (; t + 16 <= t1; t += 16) {
-      double a[16], b[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) { a[u] = w(t + u); b[u] = v(t + u); }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) acc = fma(a[u], b[u], acc);
-    }
+  if constexpr (U >= 16)
+    for (; t + 16 <= t1; t += 16) gather_batch<16, DOWN>(t, last, acc, w, v);
+  if constexpr (U >= 8)
+    for (; t + 8 <= t1; t += 8) gather_batch<8, DOWN>(t, last, acc, w, v);
+  if constexpr (U >= 4)
+    for (; t + 4 <= t1; t += 4) gather_batch<4, DOWN>(t, last, acc, w, v);
+  if constexpr (U >= 2)
+    for (; t + 2 <= t1; t += 2) gather_batch<2, DOWN>(t, last, acc, w, v);
+  if constexpr (U == 1) {  // (unrolled further by the compiler's choice: 206 registers, two waves a SIMD)
+#pragma unroll 4
+    for (; t < t1; ++t) gather_batch<1, DOWN>(t, last, acc, w, v);
+  } else if (t < t1) {
+    gather_batch<1, DOWN>(t, last, acc, w, v);
   }
-  if constexpr (U >= 8) {
-    for (; t + 8 <= t1; t += 8) {
-      double a[8], b[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) { a[u] = w(t + u); b[u] = v(t + u); }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) acc = fma(a[u], b[u], acc);
-    }
-  }
-  if constexpr (U >= 4) {
-    for (; t + 4 <= t1; t += 4) {
-      double a[4], b[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) { a[u] = w(t + u); b[u] = v(t + u); }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) acc = fma(a[u], b[u], acc);
-    }
-  }
-  if constexpr (U >= 2) {
-    for (; t + 2 <= t1; t += 2) {
-      double a0 = w(t), b0 = v(t), a1 = w(t + 1), b1 = v(t + 1);
-      acc = fma(a0, b0, acc);
-      acc = fma(a1, b1, acc);
-    }
-  }
-  for (; t < t1; ++t) acc = fma(w(t), v(t), acc);
   return acc;
 }
 
@@ -109,16 +102,18 @@ __device__ __forceinline__ double gather_fma(int t0, int t1, double acc, W w, V 
 // tail block, follow one by one.  The cell-per-wave solver computes a sum's
 // chunks on different lanes, and every solver rounds alike.
 constexpr int kChunk = 32;
-template <class M, int U, class W, class V>
-__device__ __forceinline__ double gather_sum(int t0, int th, int t1, double init, W w, V v) {
+template <class M, int U, bool DOWN = false, class W, class V>
+__device__ __forceinline__ double gather_sum(int t0, int th, int t1, double init, W w, V v,
+                                             int last = 0) {
   if constexpr (M::TAIL == 0) {
-    return gather_fma<U>(t0, t1, init, w, v);
+    return gather_fma<U, DOWN>(t0, t1, init, w, v, last);
   } else {
-    double acc = gather_fma<U>(t0, min(t0 + kChunk, th), init, w, v);
+    if (th - t0 <= kChunk) return gather_fma<U, DOWN>(t0, t1, init, w, v, last);  // one chunk: one sum
+    double acc = gather_fma<U, DOWN>(t0, t0 + kChunk, init, w, v, last);
 #pragma unroll 1
     for (int t = t0 + kChunk; t < th; t += kChunk)
-      acc = acc + gather_fma<U>(t, min(t + kChunk, th), 0.0, w, v);
-    return gather_fma<U>(th, t1, acc, w, v);
+      acc = acc + gather_fma<U, DOWN>(t, min(t + kChunk, th), 0.0, w, v, last);
+    return gather_fma<U, DOWN>(th, t1, acc, w, v, last);
   }
 }
 
@@ -503,11 +498,11 @@ __device__ void dev_solve(const CL &lu, CX x) {
     if constexpr (M::TAIL == 0) {
       acc = gather_fma<U>(kd + 1, k1, (double)x[i], [&](int k) -> double { return -(double)lu[k]; },
                           [&](int k) -> double { return x[M::lu_icol(k)]; });
-    } else {  // descending columns, term t of the row at k1 - 1 - t
+    } else {  // descending columns
       const int n = k1 - kd - 1;
-      acc = gather_sum<M, U>(0, i < M::NVAR - M::TAIL ? n : 0, n, (double)x[i],
-                             [&](int t) -> double { return -(double)lu[k1 - 1 - t]; },
-                             [&](int t) -> double { return x[M::lu_icol(k1 - 1 - t)]; });
+      acc = gather_sum<M, U, true>(0, i < M::NVAR - M::TAIL ? n : 0, n, (double)x[i],
+                                   [&](int k) -> double { return -(double)lu[k]; },
+                                   [&](int k) -> double { return x[M::lu_icol(k)]; }, k1 - 1);
     }
     x[i] = acc / (double)lu[kd];
   }
@@ -658,15 +653,18 @@ __device__ __forceinline__ int lc_batch2(DW dw, int dp, const LcLane &c, int t, 
 }
 
 // acc = (h.init_x0 ? x0 : h.init); acc = fma(-a(t), b(t), acc) over
-// [t, t1), batches as in lc_sum1 (the first carries the header): the terms
-// before th in chunks as gather_sum adds them, then those from th on.
+// [t, t1), batches as in lc_sum1 (the first carries the header): as one sum
+// where at most kChunk terms lie before th, else those in chunks as
+// gather_sum adds them, then the terms from th on.
 template <class M, int CS, class DW, class FX0, class FX2, class FA, class FB>
 __device__ __forceinline__ double lc_sum2(DW dw, int &dp, const LcLane &c, int t, const int th,
                                           const int t1, LcHead &h, FX0 x0m, FX2 x2m, FA am, FB bm) {
   double acc = 0.0, sum = 0.0;
   const int t0 = t;
+  const bool many = M::TAIL > 0 && th - t > kChunk;
+  const int tm = many ? th : t1;
   bool chunks = false;
-  const int n = th - t;
+  const int n = tm - t;
   if (n >= 16) { dp = lc_batch2<CS, 16, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 16; }
   else if (n >= 8) { dp = lc_batch2<CS, 8, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 8; }
   else if (n >= 4) { dp = lc_batch2<CS, 4, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 4; }
@@ -674,20 +672,20 @@ __device__ __forceinline__ double lc_sum2(DW dw, int &dp, const LcLane &c, int t
   else if (n == 1) { dp = lc_batch2<CS, 1, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 1; }
   else dp = lc_batch2<CS, 0, true>(dw, dp, c, t, acc, h, x0m, x2m, am, bm);
 #pragma unroll 1
-  for (int part = 0; part < 2; ++part) {  // before th, then from th on
-    const int te = part ? t1 : th;
+  for (int part = 0; part < 2; ++part) {  // before tm, then from tm on
+    const int te = part ? t1 : tm;
 #pragma unroll 1
     for (; t + 16 <= te; t += 16) {
-      if (!part) lc_chunk<M>(t - t0, chunks, sum, acc);
+      if (many && !part) lc_chunk<M>(t - t0, chunks, sum, acc);
       dp = lc_batch2<CS, 16, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm);
     }
-    if (!part && t < te) lc_chunk<M>(t - t0, chunks, sum, acc);
+    if (many && !part && t < te) lc_chunk<M>(t - t0, chunks, sum, acc);
     if (t + 8 <= te) { dp = lc_batch2<CS, 8, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 8; }
     if (t + 4 <= te) { dp = lc_batch2<CS, 4, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 4; }
     if (t + 2 <= te) { dp = lc_batch2<CS, 2, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 2; }
     if (t < te) { dp = lc_batch2<CS, 1, false>(dw, dp, c, t, acc, h, x0m, x2m, am, bm); t += 1; }
     if (!part && chunks) acc = sum + acc;
-    if (th == t1) break;
+    if (tm == t1) break;
   }
   return acc;
 }
@@ -765,8 +763,14 @@ __device__ __forceinline__ void dev_solve_c(const CL &lu, CX x, const LcLane &c)
 
 // ---------------------------------------------------------------------------
 
+// The plain solver.  fullchem: sixteen terms' operands are loaded before their
+// FMAs (gather_fma), four waves a SIMD so that a grid's 3,726 waves are all
+// resident; bound by the slot traffic.  A 238,464-cell step, cold and warm:
+// 3.45 and 1.69 s with a load at a time, 2.34 and 1.03 s so (eight terms 3 %
+// more; without the register bound 2.84 and 1.00 s); one cell cold 604 and 433 ms.
 template <class M>
-__global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
+__global__ __launch_bounds__(64, M::TAIL > 0 ? 4 : 1) void k_integrate(IntegrateArgs a) {
+  constexpr int U = M::TAIL > 0 ? 16 : 1;
   const int64_t cell = (int64_t)blockIdx.x * 64 + threadIdx.x;
   if (cell >= a.ncell) return;
   if (a.only_failed && a.only_failed[cell] >= 0) return;
@@ -812,7 +816,7 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
       if (st[2] > P.max_steps) { ierr = -6; break; }
       if ((T + 0.1 * H) == T || H <= P.roundoff) { ierr = -7; break; }
       H = min_f(H, fabs(Tend - T));
-      dev_fun<M>(Yc, fix, rct, Ascr, Fcn0);
+      dev_fun<M, U>(Yc, fix, rct, Ascr, Fcn0);
       st[0] += P.autonomous ? 1 : 2;  // non-autonomous: dF/dT by finite difference (0 with frozen rates)
       st[1] += 1;
     }
@@ -820,9 +824,9 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
     int nconsec = 0;
     bool singular = true;
     while (singular) {
-      dev_jac<M>(Yc, fix, rct, Ascr, LU, -1.0, 1.0 / (dir * H * kRosGamma1));
+      dev_jac<M, U>(Yc, fix, rct, Ascr, LU, -1.0, 1.0 / (dir * H * kRosGamma1));
       int ising;
-      if constexpr (M::TAIL > 0) ising = dev_decomp_crout<M>(LU);  // the order of the cell programs
+      if constexpr (M::TAIL > 0) ising = dev_decomp_crout<M, U>(LU);  // the order of the cell programs
       else ising = dev_decomp<M>(LU);
       st[5] += 1;
       if (ising == 0) {
@@ -849,7 +853,7 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
           }
           Ynew[i] = v;
         }
-        dev_fun<M>(Ynewc, fix, rct, Ascr, Kc);
+        dev_fun<M, U>(Ynewc, fix, rct, Ascr, Kc);
         st[0] += 1;
       } else {
         for (int i = 0; i < N; ++i) Kc[i] = Fcn0[i];
@@ -859,7 +863,7 @@ __global__ __launch_bounds__(64) void k_integrate(IntegrateArgs a) {
         if (hc != 0.0)
           for (int i = 0; i < N; ++i) Kc[i] = fma(hc, Ksc(j)[i], Kc[i]);
       }
-      dev_solve<M>(CCol{LU.p, ws}, Kc);
+      dev_solve<M, U>(CCol{LU.p, ws}, Kc);
       st[6] += 1;
     }
     // new solution, error estimate (E = (0,0,0,1): Yerr = K4), scaled norm
@@ -1097,19 +1101,25 @@ __device__ __forceinline__ bool lane_attempt(const IntegrateArgs &a, const Slot 
   };
   if constexpr (M::TAIL > 0) {
     // species l, l + 64, ... summed for each l, then the sums in l order (the
-    // cell-per-wave solver's lanes)
+    // cell-per-wave solver's lanes); EB species' loads at a time (all six took
+    // the variants without a register bound past 128 registers, three waves a
+    // SIMD for four)
+    constexpr int KS = (M::NVAR + 63) / 64, EB = U > 1 ? 3 : 1;
 #pragma unroll 1
     for (int l = 0; l < 64; ++l) {
-      constexpr int KS = (M::NVAR + 63) / 64;
-      double v[KS], qq[KS], part = 0.0;
+      double part = 0.0;
+#pragma unroll 1
+      for (int i = l; i < 64 * KS; i += 64 * EB) {
+        double v[EB], qq[EB];
 #pragma unroll
-      for (int k = 0; k < KS; ++k) err_term(min(l + 64 * k, N - 1), v[k], qq[k]);
+        for (int k = 0; k < EB; ++k) err_term(min(i + 64 * k, N - 1), v[k], qq[k]);
 #pragma unroll
-      for (int k = 0; k < KS; ++k)
-        if (l + 64 * k < N) {
-          Ynew[l + 64 * k] = v[k];
-          part = fma(qq[k], qq[k], part);
-        }
+        for (int k = 0; k < EB; ++k)
+          if (i + 64 * k < N) {
+            Ynew[i + 64 * k] = v[k];
+            part = fma(qq[k], qq[k], part);
+          }
+      }
       err += part;
     }
   } else

@@ -90,10 +90,7 @@ def lu_events(m, t):
             if q != kd:
                 ghimj(q)
             dv = t["cr_div"][q]
-            # (a tail block's own pivots follow the terms in front of it in
-            # batches of their own, cell_sched.tail_size)
-            parts = _split(list(range(t["cr_ptr"][q], t["cr_hd"][q]))) or [[]]
-            parts += _split(list(range(t["cr_hd"][q], t["cr_ptr"][q + 1])))
+            parts = _parts(list(range(t["cr_ptr"][q], t["cr_ptr"][q + 1])), t["cr_hd"][q] - t["cr_ptr"][q])
             for n_, part in enumerate(parts):
                 rd = []
                 for x in part:
@@ -101,6 +98,15 @@ def lu_events(m, t):
                 ev.append(("C", rd, [dv if dv >= 0 else None] if n_ == 0 else []))
             ev.append(("W", q))
     return ev
+
+
+def _parts(ks, nhd):
+    """Batches of a sum of two operands: after more than a chunk of terms in
+    front of the tail block (cell_sched.tail_size) its own pivots' terms have
+    batches of their own, otherwise they are one sum."""
+    if nhd <= cell_sched.CHUNK:
+        return _split(ks) or [[]]
+    return _split(ks[:nhd]) + _split(ks[nhd:])
 
 
 def solve_events(m):
@@ -114,7 +120,7 @@ def solve_events(m):
     tail = cell_sched.tail_size(m)
 
     def row(i, ks, nhd, extras):
-        for n_, part in enumerate((_split(ks[:nhd]) or [[]]) + _split(ks[nhd:])):
+        for n_, part in enumerate(_parts(ks, nhd)):
             rd = []
             for k in part:
                 rd += [k, ("x", icol[k])]

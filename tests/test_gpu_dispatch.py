@@ -215,3 +215,28 @@ def test_infinite_entries_spoil_the_same_rows_in_every_kernel(factor, inputs, fu
     for a, b in zip(*out):
         assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
     assert some.sum() > 20
+
+
+@pytest.mark.parametrize("variant", [0, 1, 4, 6, 8, 9, None])
+@pytest.mark.parametrize("n", [1, 65, 200])
+def test_every_lane_solver_adds_in_the_same_order(n, variant, inputs, fullchem, torch_dev):
+    """fullchem's lane kernels and the plain solver (None), whose gathers load
+    one to sixteen terms at a time, against the default kernel, bit by bit."""
+    from gckpp_amd import hip
+    print("case: fullchem, %d cells, lane variant %s" % (n, variant), flush=True)
+    _, conc, rct = inputs["fullchem"]
+    cells = (np.arange(n) * 37) % conc.shape[1]
+    ic, rc = options.fullchem_icntrl()
+    out = []
+    for v in (7, variant):
+        ctx = hip.Context(fullchem, max(n, 64))
+        if v is not None:
+            ctx.set_solver(hip.SOLVER_PERSISTENT)
+            ctx.set_persistent_config(v, 1)
+        c = _t(torch_dev, conc[:, cells])
+        ist, rst, ierr = ctx.integrate(c, _t(torch_dev, rct[:, cells]), _t(torch_dev, np.zeros(n)), 0.0, 1200.0, ic, rc)
+        out.append([x.cpu().numpy() for x in (c, ist, rst, ierr)])
+        ctx.close()
+    assert (out[0][3] == 1).all()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
