@@ -1505,7 +1505,9 @@ void launch_integrate_mech(int mech, const IntegrateArgs &a, hipStream_t s) {
 template <int U, int W, bool SEG, int CS = 0>
 static const void *persist_kernel(int qset) {
   switch (qset) {
-    case PQ_FULLCHEM: return (const void *)k_persist<U, W, SEG, CS, Traits_fullchem, void, void>;
+    case PQ_FULLCHEM:  // (no segments with a tail block: variants 3 and 5 run 2's and 4's code)
+      return (const void *)k_persist<U, W, SEG && Traits_fullchem::TAIL == 0, CS, Traits_fullchem, void,
+                                     void>;
     case PQ_CARBON: return (const void *)k_persist<U, W, SEG, CS, Traits_carbon, void, void>;
     case PQ_MIXED:
       return (const void *)k_persist<U, W, SEG, CS, Traits_fullchem, Traits_Hg, Traits_carbon>;

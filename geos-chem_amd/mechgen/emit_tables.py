@@ -240,9 +240,18 @@ def cell_text(name, m, t, cell):
     return "\n".join(out)
 
 
+SEGMENTS = ["cu_row", "cu_sp", "cu_q", "cu_l", "cu_u", "sf_sp", "sf_l", "sf_x", "sf_batch", "sb_sp",
+            "sb_l", "sb_x", "sb_batch"]
+
+
 def emit(name):
     m = json.loads((HERE.parent / "mech" / ("%s.json" % name)).read_text())
     t = build_tables(m)
+    # a mechanism with cell programs has no use for the flat segments (its sums
+    # go in chunks) and the block programs: their tables stay empty
+    tail = cell_sched.tail_size(m)
+    if tail:
+        t.update((k, []) for k in SEGMENTS)
     out = ["/* Generated by geos-chem_amd/mechgen/emit_tables.py from mech/%s.json"
            " -- do not edit. */" % name, "#pragma once", "",
            "namespace mech_%s {" % name,
@@ -255,15 +264,14 @@ def emit(name):
            % (max(0, len(t["sf_batch"]) - 1), max(0, len(t["sb_batch"]) - 1)), ""]
     ints = ["rx_s", "fv_ptr", "fv_r", "pt_r", "pt_s", "jv_ptr", "jv_b", "le_kk", "le_dj",
             "le_p0", "le_p1", "le_row", "lp_dst", "lp_src", "row_e0", "cr_ptr", "cr_l", "cr_u",
-            "cr_div", "cr_hd", "fw_hd", "cu_row", "cu_sp", "cu_q", "cu_l", "cu_u", "sf_sp", "sf_l", "sf_x",
-            "sf_batch", "sb_sp", "sb_l", "sb_x", "sb_batch"]
+            "cr_div", "cr_hd", "fw_hd"] + SEGMENTS
     for k in ints:
         out.append(arr("int", k, t[k]))
     for k in ("fv_c", "pt_m", "jv_c"):
         out.append(arr("double", k, t[k], per_line=6, fmt=dfmt))
     for k, key in (("lu_crow", "lu_crow"), ("lu_diag", "lu_diag"), ("lu_icol", "lu_icol")):
         out.append(arr("int", k, m[key][: (m["nvar"] + 1) if k != "lu_icol" else None]))
-    # cell-per-wave solver: LDS layout, global scratch layout and programs
+    # cell-per-wave solver: LDS layout, global scratch layout and block programs
     prog = wave_sched.build_wave_program(m, t)
     L = prog["layout"]
     out.append("constexpr int WV_ZERO = %d, WV_ONE = %d, WV_X0 = %d, WV_Y0 = %d, WV_SINK = %d, "
@@ -271,6 +279,8 @@ def emit(name):
     out.append("constexpr int WV_G_AB = %d, WV_NAB = %d, WV_G_F0 = %d, WV_G_K = %d, WV_G_SIZE = %d, "
                "WV_NCOEF = %d;" % (L["G_AB"], L["NAB"], L["G_F0"], L["G_K"], L["G_SIZE"],
                                    len(prog["coef"])))
+    if tail:
+        prog = {"coef": [0.0]}
     arrays, consts = wave_sched.emit_arrays(prog)
     have = {P for P in ("fv", "jv", "lu", "sf", "sb") if P in prog}
     cmap = dict(consts)
@@ -282,7 +292,7 @@ def emit(name):
         out.append(arr(ctype, aname, vals, per_line=6 if ctype == "double" else 16,
                        fmt=dfmt if ctype == "double" else str,
                        align=16 if aname.endswith("_ops") else 0))
-    for P in ("fv", "jv", "lu", "sf", "sb"):   # empty programs of a mechanism without an LU
+    for P in ("fv", "jv", "lu", "sf", "sb"):   # empty ones without an LU or with cell programs
         if P not in have:
             for suf in ("ops", "flag"):
                 out.append(arr("unsigned", "wv_%s_%s" % (P, suf), [0, 0, 0, 0],
@@ -294,7 +304,7 @@ def emit(name):
         lw, sw = lane_cache.build(m, t, S)
         out.append(arr("unsigned", "lc%d_lu" % S, lw + [0] * 16))
         out.append(arr("unsigned", "lc%d_sv" % S, sw + [0] * 16))
-    out.append("constexpr int TAIL = %d;" % cell_sched.tail_size(m))
+    out.append("constexpr int TAIL = %d;" % tail)
     out.append("}  // namespace mech_%s" % name)
     gen = HERE.parent / "csrc" / "gen"
     gen.mkdir(exist_ok=True)
