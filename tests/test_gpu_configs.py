@@ -1,7 +1,9 @@
 """The five benchmark workloads at their full sizes, through the C ABI.
 
-  C1  4,096 synthetic box cells (seed 0), plain and persistent steps
-  C2  the 72x46x72 grid (238,464 cells), plain and persistent steps
+  C1  4,096 synthetic box cells (seed 0), plain and persistent steps, the
+      persistent one on the default kernel and on the lane kernel with the
+      tail hand-off
+  C2  the 72x46x72 grid (238,464 cells), the same three steps
   C3  the 144x91x72 grid (943,488 cells) of fullchem, Hg and carbon cells in
       one persistent launch per step: 24 steps replayed from one captured
       HIP graph with a synthetic emission/transport perturbation between
@@ -125,7 +127,7 @@ def test_c1_golden_step_outputs(fullchem, T):
         ctx.close()
 
 
-@pytest.mark.parametrize("solver", ["plain", "persistent"])
+@pytest.mark.parametrize("solver", ["plain", "persistent", "handoff"])
 def test_c1_all_box_cells(solver, fullchem, T, refkpp):
     """C1 on all 4,096 box cells: every cell's step against the compiled
     reference's step on the same inputs."""
@@ -135,12 +137,14 @@ def test_c1_all_box_cells(solver, fullchem, T, refkpp):
     ic, rc = options.fullchem_icntrl()
     ctx = hip.Context(fullchem, w.ncell)
     ctx.set_solver(hip.SOLVER_PLAIN if solver == "plain" else hip.SOLVER_PERSISTENT)
-    if solver == "persistent":
+    if solver == "handoff":
+        ctx.set_persistent_config(4, 1)
         ctx.set_persistent_handoff(512)
     conc = _dev(T, w.conc)
     hnew, ist, ierr, ok = ctx.fullchem_step(_dev(T, w.met), _dev(T, w.photol), _dev(T, w.het), conc,
                                             _dev(T, w.hstart), DT, ic, rc)
     T.cuda.synchronize()
+    assert (ctx.handoff_stats()[0] > 0) == (solver == "handoff")
     _check_every_cell(T, fullchem, conc, hnew, ierr, "C1 " + solver)
     _vs_reference(refkpp(fullchem), fullchem, w, conc.cpu().numpy(), ist.cpu().numpy(), "C1 " + solver)
     ctx.close()
@@ -160,32 +164,38 @@ def grid72(fullchem, T):
     T.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("solver", ["plain", "persistent"])
+@pytest.mark.parametrize("solver", ["plain", "persistent", "handoff"])
 def test_c2_grid_step(solver, grid72, fullchem, T, refkpp):
     """C2: the cold 1200 s step of the 72x46x72 grid (plain one-lane-per-cell
-    solver; persistent solver with the tail hand-off of the benchmark)."""
+    solver; persistent solver on its default kernel, and on the lane kernel
+    with the tail hand-off)."""
     print("case: C2, 72x46x72 grid (238464 cells), %s step" % solver, flush=True)
     from gckpp_amd import hip
     g = grid72
     w, d, ctx, idx = g["w"], g["d"], g["ctx"], g["idx"]
     ic, rc = options.fullchem_icntrl()
     ctx.set_solver(hip.SOLVER_PLAIN if solver == "plain" else hip.SOLVER_PERSISTENT)
-    ctx.set_persistent_handoff(32768 if solver == "persistent" else 0)
+    if solver == "handoff":
+        ctx.set_persistent_config(4, 1)
+        ctx.set_persistent_handoff(32768)
     conc = d["conc0"].clone()
     cold = T.zeros(w.ncell, dtype=T.float64, device="cuda")
     hnew, ist, ierr, ok = ctx.fullchem_step(d["met"], d["photol"], d["het"], conc, cold, DT, ic, rc)
     T.cuda.synchronize()
+    if solver == "handoff":
+        assert ctx.handoff_stats()[0] > 0
+        ctx.set_persistent_handoff(0)
+        ctx.set_persistent_config(hip.WAVE_VARIANT, 1)
     _check_every_cell(T, fullchem, conc, hnew, ierr, "C2 " + solver)
     print("  mean attempts per cell %.2f" % ist[2].double().mean().item())
     _vs_reference(refkpp(fullchem), fullchem, w.subset(idx), conc[:, idx].cpu().numpy(),
                   ist[:, idx].cpu().numpy(), "C2 " + solver)
-    ctx.set_persistent_handoff(0)
 
 
 def test_c4_learned_h0_on_grid(grid72, fullchem, T, refkpp):
     """C4: the committed network's h0 and cost order on the C2 grid, the
-    persistent solver with the tail hand-off.  The reference, started from
-    the same h0 (its RCNTRL(3)), gives the same result on the sample: the
+    persistent solver.  The reference, started from the same h0 (its
+    RCNTRL(3)), gives the same result on the sample: the
     network only chooses the first step, which the controller then judges."""
     print("case: C4, learned h0 on the 72x46x72 grid", flush=True)
     from gckpp_amd import hip, learned
@@ -200,12 +210,10 @@ def test_c4_learned_h0_on_grid(grid72, fullchem, T, refkpp):
     h0, cls = model.predict(d["met"], d["photol"], conc, dt=DT)
     assert bool(((h0 >= 1e-5) & (h0 <= DT)).all().item())
     ctx.set_solver(hip.SOLVER_PERSISTENT)
-    ctx.set_persistent_handoff(32768)
     ctx.set_cell_order(hip.order_by_class(cls))
     hnew, ist, ierr, ok = ctx.fullchem_step(d["met"], d["photol"], d["het"], conc, h0.clone(), DT, ic, rc)
     T.cuda.synchronize()
     ctx.set_cell_order(None)
-    ctx.set_persistent_handoff(0)
     _check_every_cell(T, fullchem, conc, hnew, ierr, "C4 learned")
     print("  mean attempts per cell %.2f" % ist[2].double().mean().item())
     _vs_reference(refkpp(fullchem), fullchem, w.subset(idx), conc[:, idx].cpu().numpy(),
@@ -214,7 +222,7 @@ def test_c4_learned_h0_on_grid(grid72, fullchem, T, refkpp):
 
 def test_c3_mixed_grid_24_graph_replays(fullchem, hg, T, refkpp):
     """C3: 943,488 cells, fullchem/Hg/carbon 70/20/10 at random, one
-    persistent launch (with the tail hand-off) per step.  The first step's
+    persistent launch per step.  The first step's
     sample against each mechanism's compiled reference; then one captured
     step replayed 24 times with a perturbation between replays, bitwise
     equal after every step to the same 24 steps run eagerly on a copy."""
@@ -225,7 +233,6 @@ def test_c3_mixed_grid_24_graph_replays(fullchem, hg, T, refkpp):
     print("  cells per mechanism", [p.ncell for p in parts], flush=True)
     ctxs = [hip.Context(m, p.ncell) for m, p in zip(mechs, parts)]
     B = hip.Batch(*ctxs)
-    B.set_handoff(32768)
 
     def state():
         st = []
@@ -268,9 +275,9 @@ def test_c3_mixed_grid_24_graph_replays(fullchem, hg, T, refkpp):
                               s["istatus"][:, idx].cpu().numpy() if m.name != "carbon" else None,
                               "C3 first step, %s" % m.name)
         if k % 6 == 5:
-            print("  %d replays equal to the eager steps; attempts/cell %s; handed off %d"
-                  % (k + 1, [round(float(s["istatus"][2].double().mean().item()), 2) for s in graph],
-                     B.handoff_count()), flush=True)
+            print("  %d replays equal to the eager steps; attempts/cell %s"
+                  % (k + 1, [round(float(s["istatus"][2].double().mean().item()), 2) for s in graph]),
+                  flush=True)
     B.close()
     for c in ctxs:
         c.close()
@@ -280,7 +287,7 @@ def test_c3_mixed_grid_24_graph_replays(fullchem, hg, T, refkpp):
 def test_c5_c90_faces_learned_persistent(fullchem, T, refkpp):
     """C5: 6x90x90x72 = 3,499,200 cells as six face-sized chunks through one
     context whose workspace is sized for one face; learned h0, cost order,
-    persistent solver with the tail hand-off; the reference from the same
+    persistent solver; the reference from the same
     h0 on 683 strided cells of every face."""
     print("case: C5, six 90x90x72 faces (3499200 cells), learned + persistent", flush=True)
     from gckpp_amd import hip, learned, synth
@@ -291,7 +298,6 @@ def test_c5_c90_faces_learned_persistent(fullchem, T, refkpp):
     nface = 90 * 90 * 72
     ctx = hip.Context(fullchem, nface)
     ctx.set_solver(hip.SOLVER_PERSISTENT)
-    ctx.set_persistent_handoff(32768)
     model = learned.StepModel(fullchem).load(path)
     idx = _strided(nface, 683)
     wsamp, csamp, ssamp, hsamp = [], [], [], []

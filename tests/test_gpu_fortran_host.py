@@ -65,8 +65,9 @@ def _read_result(path, m, n):
                                                                 ("persistent", False, 100)])
 def test_fortran_host_step_equals_device_step(solver_name, het_per_cell, handoff, fullchem,
                                               torch_dev, tmp_path):
-    """(handoff: the host-pointer calls with the tail hand-off of the last
-    100 cells of each chunk's persistent launch.)"""
+    """(handoff: the host-pointer call through Python on the lane kernel with
+    the tail hand-off of the last 100 cells of each chunk's launch, the
+    Fortran host's with the setting, which its default kernel has no use for.)"""
     print("case: Fortran host step, %s solver, per-cell HetState %s, hand-off %d, 600 cells in "
           "chunks of 256" % (solver_name, het_per_cell, handoff), flush=True)
     from gckpp_amd import hip, synth
@@ -92,12 +93,15 @@ def test_fortran_host_step_equals_device_step(solver_name, het_per_cell, handoff
     # the host-pointer step through the Python binding, chunked
     ctx2 = hip.Context(m, 256)
     ctx2.set_solver(solver)
+    if handoff:
+        ctx2.set_persistent_config(4, 1)
     ctx2.set_persistent_handoff(handoff)
     c2 = np.ascontiguousarray(w.conc.copy())
     h2, i2, e2, ok2 = ctx2.fullchem_step_host(np.ascontiguousarray(w.met),
                                               np.ascontiguousarray(w.photol), het, c2, w.hstart,
                                               dt, ic, rc)
     assert ok2
+    assert (ctx2.handoff_stats()[0] > 0) == (handoff > 0)
     for x, y in zip(want, (c2, h2, i2, e2)):
         assert np.array_equal(x, y)
     ctx.close()

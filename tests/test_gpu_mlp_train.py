@@ -1,9 +1,12 @@
 """The training kernels at the edges of their tiles: batches of one sample,
 around the 16-sample workgroups and the 128-row chunks of the weights'
 gradients, and one past the most chunks, against the float64 oracle
-(oracle/mlp.py).  Bound: sums of up to 16,385 fp32 terms in partial sums of at
-most 32 rows of four add no more than 64 roundings in a row, 64 * 6e-8 = 4e-6
-of the sums of magnitudes, which are at most 10 times the gradient's norm."""
+(oracle/mlp.py).  Bound: a term of a weight's gradient of up to 8,197 rows goes
+through one product, at most 33 steps of four additions in its chunk (132 rows)
+and at most 63 additions of chunks, 196 roundings of 6e-8.  Independent ones
+leave sqrt(196) * 6e-8 = 8.4e-7 of the sums of magnitudes, which are up to 5
+times the gradient's norm here: 4.2e-6; the tolerance leaves ten times that for
+the activations' and the loss's own errors."""
 import numpy as np
 import pytest
 

@@ -401,7 +401,9 @@ def test_split_persistent_step_bitwise(name, forced, mech_of, torch_dev):
     """The split persistent step -- the first cells of the h0 order on the
     cell-per-wave kernel on a second stream, the rest on the lane kernel at
     the same time -- gives bitwise the single-kernel step's results, also
-    when cells fail and take the retry."""
+    when cells fail and take the retry.  (A lane variant is chosen: without
+    a choice fullchem runs the cell-per-wave kernel alone and Hg the lane
+    kernel alone.)"""
     print("case: split persistent step, %s, forced retries %s" % (name, forced), flush=True)
     from gckpp_amd import hip, synth
     from gckpp_amd.options import icntrl_for
@@ -421,8 +423,10 @@ def test_split_persistent_step_bitwise(name, forced, mech_of, torch_dev):
     for split in (0, 150):
         ctx = hip.Context(m, 2048)
         ctx.set_solver(hip.SOLVER_PERSISTENT)
+        ctx.set_persistent_config(4, 1)
         ctx.set_cell_order(order)
         ctx.set_persistent_split(split)
+        assert ctx.persistent_config()["wave_per_cell"] == 0
         conc = _t(T, w.conc)
         hnew, ist, ierr, ok = ctx.fullchem_step(_t(T, w.met), _t(T, w.photol), _t(T, w.het), conc,
                                                 _t(T, hs), 1200.0, ic, rc)
