@@ -464,8 +464,8 @@ def end_to_end(args, w, ctx, ic, rc):
     """The same cold step from host arrays through gckpp_fullchem_step (the
     Fortran host's call): the inputs copied to the device, the step, the
     results copied back, all inside the timed region.  Persistent solver
-    with the context's hand-off, Hstart = 0 (a host-pointer call takes no
-    cell order or predicted h0), pageable host memory; the first call
+    (on a lane variant with the context's hand-off), Hstart = 0 (a host-pointer
+    call takes no cell order or predicted h0), pageable host memory; the first call
     allocates the staging buffers and is not timed."""
     import numpy as np
     from gckpp_amd import hip
@@ -487,8 +487,8 @@ def end_to_end(args, w, ctx, ic, rc):
     return {"value": round(w.ncell / wall, 2), "unit": "cells/s", "ms_per_step": round(wall * 1e3, 3),
             "calls": nrep, "ms_min": round(min(tim) * 1e3, 3), "ms_max": round(max(tim) * 1e3, 3),
             "host_bytes_moved": int(nbytes), "failed_cells": int((ierr < 0).sum()),
-            "path": "host arrays -> gckpp_fullchem_step (staged H2D, persistent solve with the "
-                    "hand-off, D2H), Hstart 0, pageable memory"}
+            "path": "host arrays -> gckpp_fullchem_step (staged H2D, persistent solve, D2H), "
+                    "Hstart 0, pageable memory"}
 
 
 def warm_legs(args, mech, w, ctx, model, P, ic, rc):

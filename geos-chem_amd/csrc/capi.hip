@@ -166,12 +166,14 @@ static int set_pconfig(gckpp_ctx *c, int variant, int wpb) {
 
 // Scratch of gckpp_integrate_noalloc_dev: the work-stealing counter
 // (the first 256 bytes) and the blocks of up to kNoAllocWaves waves of the
-// cell-per-wave solver (each wave's rate constants, reaction products,
-// Fcn0 and stage vectors: wave_scratch_fields(mech) fields of 64 doubles,
-// 73 for fullchem, the largest).  768 waves are three fullchem cells per
-// CU on 256 CUs; 28 MiB per device, held until the process ends.  Host
-// code reaches each device's copy through the address that
-// hipGetSymbolAddress gives with that device current (g_na_ptr), never
+// cell-per-wave solver: wave_scratch_fields(mech) fields of 64 doubles a wave,
+// 73 for fullchem, the largest.  The block programs (Hg, carbon) keep a wave's
+// rate constants, reaction products, Fcn0 and stage vectors there; the cell
+// programs (fullchem) keep them in registers and LDS and leave their block
+// unused, which still limits the waves a call may ask for.  768 waves are
+// three fullchem cells per CU on 256 CUs; 28 MiB per device, held until the
+// process ends.  Host code reaches each device's copy through the address
+// that hipGetSymbolAddress gives with that device current (g_na_ptr), never
 // through the array's name.
 constexpr int64_t kNoAllocWaves = 768, kNoAllocFields = 73, kNoAllocHead = 32;
 constexpr int64_t kNoAllocDoubles = kNoAllocHead + kNoAllocWaves * kNoAllocFields * 64;

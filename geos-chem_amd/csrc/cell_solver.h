@@ -14,7 +14,7 @@
 // substitutions read it, a step's lanes side by side (112 ms without).
 // Measured on the 24x23x72 grid, cold step of 39,744 cells: 537 ms with the
 // block programs of wave_sched.py, 101 ms here; 55 us an attempt and wave where
-// it was 280 us; one cell's Integrate 9.2 ms and 2.3 ms.
+// it was 280 us; one cell's Integrate 9.1 ms and 2.2 ms.
 //
 // Included by wave_solver.hip inside namespace gckpp.
 #pragma once

@@ -6,11 +6,13 @@
 // The table walk reads every operand from the wave's slot block in memory, a
 // wait every few FMAs; a Hg cell is 161 LU entries and 32 species, and an
 // attempt about 4,000 FP64 instructions.  Here they are that many instructions
-// on values that stay on the CU: the diagonal and the vectors in registers, the
-// other LU entries and the fixed species in 80 KB of LDS a wave.  So two waves a
-// CU; with four (40 KB each, the LU in registers) the compiler spilled 200 to
-// 500 values and the spills' way to memory bounded the kernel (21.6 ms of the
-// step below).  Lanes take new cells from the counter sixteen at a time: a
+// on values that mostly stay on the CU: the diagonal and the vectors in 512
+// registers, the other LU entries and the fixed species in 80 KB of LDS a wave.
+// What does not fit goes to memory: the state and 74 rate constants to the slot
+// block, 162 of the values between the partials and the LU to scratch (376
+// bytes a lane).  So two waves a CU; with four (40 KB each, the LU in registers)
+// the compiler spilled 200 to 500 values and the spills' way to memory bounded
+// the kernel (21.6 ms of the step below).  Lanes take new cells from the counter sixteen at a time: a
 // refill's loads wait once for all of them.
 // Measured on the 72x46x72 grid (238,464 Hg cells, cold step): 38.1 ms with the
 // table walk, 11.9 ms here, 70 us an attempt and wave, two thirds of it waiting

@@ -95,7 +95,8 @@ int gckpp_integrate_dev(gckpp_ctx *ctx, int64_t ncell, double tin, double tout,
  * capture, tight serving loops).  Same arguments and results (bitwise) as
  * gckpp_integrate_dev with the persistent solver's cell-per-wave variant;
  * any ncell.  Its scratch is a static device array of 28 MiB per device
- * (the work-stealing counter and up to 768 fullchem waves), reserved when
+ * (the work-stealing counter and the waves' blocks, for at most 768 fullchem
+ * waves), reserved when
  * the library is loaded and held until the process ends; the call itself
  * makes no hipMalloc or other allocation.  Fails with a message when the
  * context's wave cap (gckpp_set_persistent_waves) asks for more waves than
@@ -307,7 +308,11 @@ int gckpp_step_timings(gckpp_ctx *ctx, float ms[4]);
  * Variants 8, 9: one lane per cell with an operand cache of C = 16 / 32
  * values per lane in LDS for the LU and the substitutions, managed by a
  * schedule computed when the mechanism is compiled ((16,4,0), (16,2,0)).
- * All variants add the same terms in the same order.  get: out = {variant,
+ * All variants add the same terms in the same order.  fullchem has no flat
+ * segment lists: its variants 3 and 5 run the code of 2 and 4.  Hg runs one
+ * kernel for every lane variant (0-6, 8, 9): a lane's cell in registers and
+ * LDS, straight-line code, one wave per workgroup.  A fullchem context starts
+ * on variant 7, an Hg or carbon context on variant 4.  get: out = {variant,
  * waves_per_group, waves per launch, U, W, S, C}. */
 int gckpp_persistent_variants(void);
 int gckpp_set_persistent_config(gckpp_ctx *ctx, int variant, int waves_per_group);
@@ -324,16 +329,19 @@ int gckpp_set_cell_order(gckpp_ctx *ctx, const int32_t *order);
 int gckpp_set_step_log(gckpp_ctx *ctx, float *hlog, int nattempt);
 
 /* Split persistent solve (no reference counterpart).  With nfirst > 0 and a
- * cell order set, the next persistent Integrate or step runs the first
- * nfirst cells of the order on the cell-per-wave kernel (variant 7) on a
+ * cell order set, a persistent Integrate or step on a lane variant runs the
+ * first nfirst cells of the order on the cell-per-wave kernel (variant 7) on a
  * second stream of the context, concurrently with the configured variant on
  * the rest of the order; the call's stream waits for both.  Meant for the
  * costliest cells of an uneven step (a warm step, cells ordered by
  * gckpp_order_by_h0_dev): one cell-per-wave attempt takes far less time than
  * a lane-per-cell attempt, so the longest chains of attempts stop setting
  * the step's length.  Results are bitwise those of one kernel.  0 turns it
- * off; ignored without a cell order, for carbon and when nfirst >= ncell.
- * The first call with nfirst > 0 allocates the cell-per-wave slots. */
+ * off; ignored without a cell order, for carbon, when nfirst >= ncell, on
+ * variant 7 (so on a fullchem context that was not configured: its cells are
+ * all on that kernel) and on an Hg context that was not configured with
+ * gckpp_set_persistent_config (64 cells a wave beat one).  The first call
+ * with nfirst > 0 allocates the cell-per-wave slots. */
 int gckpp_set_persistent_split(gckpp_ctx *ctx, int64_t nfirst);
 
 /* Cap on the waves of a persistent launch (no reference counterpart): at
@@ -353,7 +361,9 @@ int gckpp_set_persistent_waves(gckpp_ctx *ctx, int64_t max_waves);
  * takes far less time on the cell-per-wave kernel than on a lane whose wave
  * is otherwise idle, so the last cells stop setting the step's length.
  * Results are bitwise those without the hand-off.  0 turns it off; not for
- * carbon.  A call with a larger max_cells than before allocates the list
+ * carbon.  Like the split it has no effect on variant 7 and on an Hg context
+ * that was not configured with gckpp_set_persistent_config.  A call with a
+ * larger max_cells than before allocates the list
  * ((15 + NVAR) doubles and one int per cell) and, the first time, the
  * cell-per-wave scratch. */
 int gckpp_set_persistent_handoff(gckpp_ctx *ctx, int64_t max_cells);
@@ -361,8 +371,8 @@ int gckpp_set_persistent_handoff(gckpp_ctx *ctx, int64_t max_cells);
  * attempts the cell-per-wave launch made on them; ms[0] the lane launch's
  * duration, ms[1] the cell-per-wave launch's (HIP events on the call's
  * stream).  All zeros when the last solve ran no hand-off (plain solver,
- * hand-off off, carbon, the cell-per-wave variant) or before the first
- * solve.  Synchronises the device. */
+ * hand-off off or without effect) or before the first solve.  Synchronises
+ * the device. */
 int gckpp_persistent_handoff_stats(gckpp_ctx *ctx, int64_t n[2], float ms[2]);
 
 /* Autotuner: integrates a copy of the given cells with every persistent
